@@ -156,28 +156,39 @@ __global__ void __launch_bounds__(GP_T) k_gather_push(const double* __restrict__
 
 // ------------------------------------------------------------------ fused push + deposition
 //
-// One block takes PPT consecutive particles per thread (thread t owns
-// particles p0 + t*PPT + j, so the lanes of a wave sit PPT particles
-// apart and, with particles in cell order, mostly in different cells).
-// Phase 1 optionally pushes positions (particle_tools.f90:58-82) and finds the
-// block's cell bounding box for J (at the half-step positions) and rho (at the
-// new positions).  Then, one component (J_x, J_y, J_z, rho) at a time, the
-// block accumulates into an LDS tile covering the box with LDS FP64 atomics
-// and hands the tile on:
-//  * a block whose tile spans at most DEP_SLOT_R node rows and 8*PPT node
-//    columns (the common case for particles in the reference's generation
-//    order or sorted by cell: 512 particles cover about 32 cells of one or two
-//    cell rows) stores its tile with plain stores in a slot of its own and
-//    records (first node row, first node column, width, rows) in a
-//    descriptor; k_dep_combine then adds the slots into the grid, so no
-//    global atomics;
-//  * any other block adds its tile to the grid with one global atomic per
-//    node and component, and a box too large for the LDS budget makes the
-//    block deposit straight to the grid with global atomics, one per node
-//    value and cell from the same per-cell register sums (a block that spans
-//    the end of one cell row and the start of the next is such a block).
+// A block of four waves takes a group of DEP_T * PPL consecutive particles, PPL
+// per lane:
+//  1. Every lane loads its particles once (coalesced), pushes them
+//     (particle_tools.f90:58-82), finds their cells, weights and phases for J
+//     (half-step positions) and rho (new positions), and leaves J's in LDS for
+//     its wave; the block reduces the node bounding box of both deposits.
+//  2. Each wave cuts its particles into segments of one cell, listed in LDS
+//     from ballots.  A lane takes one (segment, component, node row of the
+//     cell): it sums the particles of the segment on the row's two nodes, all
+//     modes, in FP64 registers and adds the sums to the block's LDS tile (real
+//     planes: Re of mode 0, then Re and Im of each mode) with ds_add_f64.  rho
+//     follows J through the same LDS.
+//  3. The block hands the tile on:
+//      * a tile of at most DEP_SLOT values goes with plain stores, as it is,
+//        into the group's own slot, with a descriptor (first node row, first
+//        node column, width, rows); k_dep_combine then adds the slots into the
+//        grid, so no global atomics;
+//      * a larger tile is added to the grid with one global atomic per node
+//        value; the planes take as many passes as the LDS needs (all four
+//        components at once, J then rho, or one component at a time);
+//      * a box with no room even for one component's planes (a group that
+//        spans the end of one cell row and the start of the next) sends each
+//        segment's sums to the grid with global atomics.
 // Deposits are unfolded; the forward FB transform applies the ghost fold.
-
+//
+// What bounds it: about equally the 104 bytes per particle in and out of HBM
+// (with the slots 8.9 GB of traffic for 67.0 M electrons at four modes), the
+// segments' arithmetic and their LDS reads and adds; three blocks of a CU share
+// them.  There it takes 2.8 ms, and the combine 0.9; one pass per component over
+// particles re-read from memory (46 GB) took 5.5, with a combine of 1.2.  Mixed
+// precision, 16.7 M at three modes: 0.75 + 0.11 ms, before 1.24 + 0.13 and 70 us
+// to sort the slots.  (Loading the next group during the deposit of one, a
+// block taking several, changed nothing: the other blocks already hide it.)
 
 template <typename RT>
 struct DepArgsT {
@@ -193,431 +204,519 @@ struct DepArgsT {
     GridGeom gJ, gR;    // geometry for J (leftX at the current deposit) and rho
     C* J;               // (nx+1, nr+1, M, 3) or null
     C* R;               // (nx+1, nr+1, M) or null
-    C* slotJ;           // [block][3*M][DEP_SLOT_R][8*PPT] (with J)
-    C* slotR;           // [block][M][DEP_SLOT_R][8*PPT] (with R)
-    int4* desc;         // [2][blocks]: (first node row or -1, first node column, width, rows) of J, then of R
-    int nblocks;
-    int vec4;           // particle arrays allow 32-byte vector access (ld % 4 == 0, 32-byte aligned bases)
+    RT* slot;           // [group][DEP_SLOT]: J's components, then rho, each 2M-1 planes of width * rows
+                        // values, starting on an even value
+    int4* desc;         // [group]: (first node row or -1, first node column, width, rows)
+    uint32_t* mask;     // [nr+1][words]: bit b of a node row: a slot of groups 64b..64b+63 covers it (nullable)
+    int words;          // 32-bit words per row of mask
+    int ngroups;
+    int vec;            // particle arrays allow PPL-wide vector access (ld % PPL == 0, aligned bases)
 };
 
-typedef double dv4 __attribute__((ext_vector_type(4)));
-typedef float fv4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ dv4 ld4(const double* p) { return *reinterpret_cast<const dv4*>(p); }
-__device__ __forceinline__ fv4 ld4(const float* p) { return *reinterpret_cast<const fv4*>(p); }
-__device__ __forceinline__ void st4(double* p, dv4 v) { *reinterpret_cast<dv4*>(p) = v; }
-
-// A thread owns PPT consecutive particles, handled in groups of DEP_G (one
-// 32-byte vector load per component and group).
-constexpr int DEP_THREADS = 64, DEP_G = 4;
-// LDS tile of a block: one component (J_x, J_y, J_z or rho) at a time, all
-// modes, complex FP64: 16 KiB hold 1024 / nmod nodes -- the 33 x 3 nodes of 512
-// cell-ordered particles at 16 per cell up to nmod = 4 -- and eight blocks per
-// CU use 128 of the 160 KiB of LDS.  Eight particles per thread (512 per
-// block) with 64-column slots: at lpa_cfg2 on cell-sorted particles the
-// deposit takes 6.9 ms per FP64 step against 7.5 ms with four per thread and
-// 32-column slots (with those slots, eight per thread had overflowed them into
-// global atomics and measured slower).
-constexpr int DEP_LDS_BYTES = 16 * 1024;
-constexpr int DEP_SLOT_R = 4;   // node rows of one slot; its columns: 8 per particle of a thread
-// Particles per thread (PPT) by launch: 8 (512 per block, 64-column slots) when
-// the particles average at least 8 per cell, else 4 (256 per block, 32-column
-// slots): a sparse bunch's 512 particles span more columns than a slot holds.
+constexpr int DEP_T = 256, DEP_WAVES = DEP_T / 64;
+// LDS tile in doubles: with the particle data of PPL = 2 (32 KiB) three blocks
+// fill the 160 KiB of a CU (allocated 1280 bytes at a time).  At four modes it
+// holds J and rho on 85 nodes (512 cell-sorted particles at 16 per cell span
+// 33 x 2), J on 114 (in the lattice's own order they span 33 x 3).
+constexpr int DEP_POOL = 2400;
+// values of a slot: at two modes 341 nodes, more than the 65 x 4 of a sparse
+// bunch's 256 particles (4 per cell, drifting over a row boundary)
+constexpr int DEP_SLOT = 4096;
+constexpr uint32_t DEP_SKIP = 0xFFFFFFFFu;
 
 __device__ __forceinline__ void lds_add(double* p, double v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ __forceinline__ void lds_add(float* p, float v) {
-    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+
+// LDS written by some lanes of a wave and read by others of the same wave
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ bool cell_of(double xp, double yp, double zp, const GridGeom& g, int& ix, int& ir) {
-    const double rp = sqrt(yp * yp + zp * zp);
-    if (!(rp < g.rmax)) return false;
+// Minimum / maximum over a wave, in lane 63 (row shifts and row broadcasts; a
+// lane without a source keeps its own value).
+template <bool MAX>
+__device__ __forceinline__ int wave_reduce63(int v) {
+    auto op = [](int a, int b) { return MAX ? max(a, b) : min(a, b); };
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));
+    v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));
+    return v;
+}
+
+// g = sqrt(a) and h = 1/sqrt(a) for a in [1e-280, 1e300], to about one unit in
+// the last place: the hardware estimate (23 bits) refined by two coupled
+// Newton steps (Goldschmidt's form), and a residual correction of g.
+__device__ __forceinline__ void sqrt_rsqrt(double a, double& g, double& h) {
+    const double y = __builtin_amdgcn_rsq(a);
+    g = a * y;
+    h = 0.5 * y;
+    double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, a), h, g);
+    h = h + h;
+}
+
+// Cell (ix, ir), linear weights s = (x, r) of the upper nodes and phase
+// p1 = (y - i z)/r (0 at r = 0) of one particle (grid_deps.f90:41-66), under
+// the conditions of part_geom.
+__device__ __forceinline__ bool dep_geom(double xp, double yp, double zp, const GridGeom& g, int& ix, int& ir,
+                                         double2& s, double2& p1) {
+    const double r2 = yp * yp + zp * zp;
+    double rp, inv;
+    sqrt_rsqrt(r2, rp, inv);
+    if (!(r2 >= 1e-280)) {          // on the axis, or not a number
+        rp = sqrt(r2);
+        inv = rp > 0.0 ? 1.0 / rp : 0.0;
+    }
     const double fx = (xp - g.leftX) * g.dx_inv, fr = (rp - g.r0) * g.dr_inv;
-    if (!(fx >= 0.0 && fx < (double)g.nx) || !(fr >= 0.0 && fr < (double)g.nr)) return false;
-    ix = (int)floor(fx);
-    ir = (int)floor(fr);
+    if (!(rp < g.rmax) || !(fx >= 0.0 && fx < (double)g.nx) || !(fr >= 0.0 && fr < (double)g.nr)) return false;
+    const double fix = floor(fx), fir = floor(fr);
+    ix = (int)fix;
+    ir = (int)fir;
+    s = cmk(fx - fix, (rp - g.Rgrid[ir]) * g.dr_inv);
+    p1 = cmk(yp * inv, -zp * inv);
     return true;
 }
 
+// One wave's LDS: its particles' weights, phases, charges and cells, and its
+// segments.  Particle p sits at p + p/16: cells of 16 particles would otherwise
+// start on one bank.
+template <int PPL>
+struct DepWave {
+    static constexpr int WP = 64 * PPL, N = WP + WP / 16;
+    double2 s[N], p1[N];
+    double q[3][N + 7];
+    uint32_t cell[WP];
+    uint16_t seg[WP + 8];
+    __device__ static int pos(int p) { return p + (p >> 4); }
+};
 
-// R: precision of momenta, weights and grids (double, or float in mixed
-// precision).  Positions, the push and the cell geometry stay FP64; each
-// corner contribution is formed and summed per cell in FP64, and the LDS tile
-// is FP64 in both precisions (FP64 LDS atomics measured far cheaper here than
-// FP32 ones under this access pattern), rounded to R when it leaves the block.
-template <int NMOD, typename R, int PPT>
-__global__ void __launch_bounds__(DEP_THREADS) k_push_deposit(DepArgsT<R> a) {
-    constexpr int SW = 8 * PPT;   // slot columns
-    typedef cplx_t<R> C;
-    constexpr int DEP_CHUNK = DEP_THREADS * PPT;
-    __shared__ double tile[DEP_LDS_BYTES / sizeof(double)];
-    __shared__ int red[8][DEP_THREADS / 64];
-    __shared__ int box[8];
-    const int tid = threadIdx.x;
-    const int blk = xcd_block(blockIdx.x, gridDim.x);
-    const GridGeom gJ = frame_geom(a.gJ), gR = frame_geom(a.gR);
-    const int64_t p0 = (int64_t)blk * DEP_CHUNK;
-    constexpr int nmod = NMOD;
-    const int64_t ld = a.ld;
-    const bool doJ = a.J != nullptr, doR = a.R != nullptr;
+// Segments of the wave's particles (keys of this lane's PPL particles in key):
+// cut at every change of cell and every `run` particles, with the shortest run
+// that keeps all (segment, component, node row) triples in one round of the 64
+// lanes.  Returns their number; seg[i] is the first particle of segment i,
+// seg[number] = WP.
+template <int PPL, int NCOMP>
+__device__ __forceinline__ int dep_segments(DepWave<PPL>& L, const uint32_t (&key)[PPL]) {
+    constexpr int BUDGET = 32 / NCOMP, WP = DepWave<PPL>::WP;
+    const int lane = threadIdx.x & 63;
+    const uint64_t below = (1ull << lane) - 1ull;
+    uint32_t prev = (uint32_t)__builtin_amdgcn_update_dpp((int)DEP_SKIP, (int)key[PPL - 1], 0x138, 0xf, 0xf, false);
+    bool head[PPL];
+    int nh = 0;
+#pragma unroll
+    for (int k = 0; k < PPL; k++) {
+        head[k] = key[k] != prev;
+        prev = key[k];
+        nh += __popcll(__ballot(head[k]));
+    }
+    int run = 4, inv = 65536 / 4;                 // p / run = (p * inv) >> 16 for p < 128
+    while (run < WP && nh + (((WP - 1) * inv) >> 16) > BUDGET) {
+        run += run >> 1;
+        inv = (65536 + run - 1) / run;
+    }
+    int nseg = 0, at = 0;
+#pragma unroll
+    for (int k = 0; k < PPL; k++) {
+        const int p = lane * PPL + k;
+        head[k] = head[k] || p == ((p * inv) >> 16) * run;
+        const uint64_t b = __ballot(head[k]);
+        nseg += __popcll(b);
+        at += __popcll(b & below);
+    }
+#pragma unroll
+    for (int k = 0; k < PPL; k++) {
+        const int p = lane * PPL + k;
+        L.cell[p] = key[k];
+        if (head[k]) L.seg[at++] = (uint16_t)p;
+    }
+    if (lane == 0) L.seg[nseg] = (uint16_t)WP;
+    wave_lds_fence();
+    return nseg;
+}
 
-    // ---- phase 1: load the thread's PPT consecutive particles, DEP_G at a
-    // time (32-byte vector loads when the arrays allow: with PPT = DEP_G a
-    // wave then reads 2 KB contiguous per component), push, store, bounding
-    // boxes.
-    const int64_t ib0 = p0 + (int64_t)tid * PPT;
-    // group h of the thread's particles: component c of array p at particle ib0 + h*DEP_G + j
-    auto load_parts = [&](const auto* p, double (&v)[3][DEP_G], int ncomp, int h) __attribute__((always_inline)) {
-        const int64_t ib = ib0 + h * DEP_G;
-        if (a.vec4 && ib + DEP_G <= a.np) {
+// The wave's segments into components c0..c0+NCP-1 (charges L.q[c0..]): to the
+// tile (pns values per component: planes of nn nodes, rows of TX; key = node of
+// the cell's lower corner), or, untiled, straight to the grid (key = node offset in a mode plane).  The
+// lanes of one ds_add_f64 add to different nodes.  (With all four corners in a
+// lane the segments had to be cut shorter to fill the lanes, and several of one
+// cell collided on every add.)
+template <int NMOD, int NCP, int PPL, typename R>
+__device__ __forceinline__ void dep_pass(DepWave<PPL>& L, int nseg, int c0, bool tiled, double* tile, int pns, int nn,
+                                         int TX, cplx_t<R>* grid, int64_t sr, int64_t sm, int64_t sl) {
+    constexpr int PL = 2 * NMOD - 1;
+    for (int t = threadIdx.x & 63; t < nseg * (2 * NCP); t += 64) {
+        const int sg = t / (2 * NCP), rem = t - sg * (2 * NCP), c = rem >> 1;
+        const bool up = rem & 1;
+        const int pb = L.seg[sg], pe = L.seg[sg + 1];
+        const uint32_t key = L.cell[pb];
+        if (key == DEP_SKIP) continue;
+        const double* q = L.q[c0 + c];
+        double acc[PL][2];
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                if (c >= ncomp) break;
-                const auto t = ld4(p + c * ld + ib);
-                v[c][0] = t.x, v[c][1] = t.y, v[c][2] = t.z, v[c][3] = t.w;
-            }
-        } else {
+        for (int i = 0; i < PL; i++) acc[i][0] = acc[i][1] = 0.0;
+        for (int p = pb; p < pe; p++) {
+            const int o = DepWave<PPL>::pos(p);
+            const double2 s = L.s[o], p1 = L.p1[o];
+            const double qp = q[o] * (up ? s.y : 1.0 - s.y);
+            const double w0 = 1.0 - s.x, w1 = s.x;
+            acc[0][0] += w0 * qp;
+            acc[0][1] += w1 * qp;
+            double2 pv = crs(qp, p1);
 #pragma unroll
-            for (int j = 0; j < DEP_G; j++)
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    if (c >= ncomp) break;
-                    v[c][j] = ib + j < a.np ? p[c * ld + ib + j] : 0.0;
-                }
-        }
-    };
-    int bx[8] = {INT_MAX, INT_MIN, INT_MAX, INT_MIN, INT_MAX, INT_MIN, INT_MAX, INT_MIN};
-    for (int h = 0; h < PPT / DEP_G; h++) {
-    const int64_t ib = ib0 + h * DEP_G;
-    const bool full = a.vec4 && ib + DEP_G <= a.np;
-    double X[3][DEP_G], XH[3][DEP_G], U[3][DEP_G], W[3][DEP_G];   // W: row 0 only
-    load_parts(a.x, X, 3, h);
-    load_parts(a.u, U, 3, h);
-    load_parts(a.w, W, 1, h);
-    if (!a.push) load_parts(a.xh, XH, 3, h);
-    if (a.push) {
-        // particle_tools.f90:58-82: x += u*dt/gamma; x_half = (x_old + x_new)/2
-#pragma unroll
-        for (int j = 0; j < DEP_G; j++) {
-            const double dt_gp = a.dt / sqrt(1.0 + (U[0][j] * U[0][j] + U[1][j] * U[1][j] + U[2][j] * U[2][j]));
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const double xn = X[c][j] + U[c][j] * dt_gp;
-                XH[c][j] = 0.5 * (X[c][j] + xn);
-                X[c][j] = xn;
+            for (int m = 1; m < NMOD; m++) {
+                acc[2 * m - 1][0] += w0 * pv.x;
+                acc[2 * m - 1][1] += w1 * pv.x;
+                acc[2 * m][0] += w0 * pv.y;
+                acc[2 * m][1] += w1 * pv.y;
+                if (m + 1 < NMOD) pv = cmul(pv, p1);
             }
         }
-        if (full) {
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                st4(a.x + c * ld + ib, dv4{X[c][0], X[c][1], X[c][2], X[c][3]});
-                st4(a.xh + c * ld + ib, dv4{XH[c][0], XH[c][1], XH[c][2], XH[c][3]});
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < DEP_G; j++) {
-                const int64_t ip = ib + j;
-                if (ip >= a.np) break;
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    a.x[c * ld + ip] = X[c][j];
-                    a.xh[c * ld + ip] = XH[c][j];
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < DEP_G; j++) {
-        if (W[0][j] == 0.0) continue;
-        int ix, ir;
-        if (doJ && (fabs(U[0][j]) + fabs(U[1][j]) + fabs(U[2][j])) != 0.0 &&
-            cell_of(XH[0][j], XH[1][j], XH[2][j], gJ, ix, ir)) {
-            bx[0] = min(bx[0], ix); bx[1] = max(bx[1], ix); bx[2] = min(bx[2], ir); bx[3] = max(bx[3], ir);
-        }
-        if (doR && cell_of(X[0][j], X[1][j], X[2][j], gR, ix, ir)) {
-            bx[4] = min(bx[4], ix); bx[5] = max(bx[5], ix); bx[6] = min(bx[6], ir); bx[7] = max(bx[7], ir);
-        }
-    }
-    }
-    for (int q = 0; q < 8; q++) {
-        const int v = (q & 1) ? wave_max(bx[q]) : wave_min(bx[q]);
-        if ((tid & 63) == 0) red[q][tid >> 6] = v;
-    }
-    __syncthreads();
-    if (tid < 8) {
-        int v = red[tid][0];
-        for (int wv = 1; wv < DEP_THREADS / 64; wv++) v = (tid & 1) ? max(v, red[tid][wv]) : min(v, red[tid][wv]);
-        box[tid] = v;
-    }
-    __syncthreads();
-    // tiles: one component at a time, (TX x TR nodes) x nmod modes, complex = 2 doubles
-    const int TXJ = box[1] >= box[0] ? box[1] - box[0] + 2 : 0, TRJ = box[3] >= box[2] ? box[3] - box[2] + 2 : 0;
-    const int TXR = box[5] >= box[4] ? box[5] - box[4] + 2 : 0, TRR = box[7] >= box[6] ? box[7] - box[6] + 2 : 0;
-    const int64_t nJ = (int64_t)TXJ * TRJ * nmod * 2, nR = (int64_t)TXR * TRR * nmod * 2;
-    const bool tileJ = doJ && nJ > 0 && nJ * (int64_t)sizeof(double) <= DEP_LDS_BYTES;
-    const bool tileR = doR && nR > 0 && nR * (int64_t)sizeof(double) <= DEP_LDS_BYTES;
-    const bool slotJ = tileJ && TRJ <= DEP_SLOT_R && TXJ <= SW;
-    const bool slotR = tileR && TRR <= DEP_SLOT_R && TXR <= SW;
-
-    // ---- phases 2 and 3, one pass per component (J_x, J_y, J_z, rho): zero
-    // the tile, deposit into it, then write it to the block's slot (a tile no
-    // taller than DEP_SLOT_R rows and no wider than SW columns) or add
-    // it to the grid with global atomics.  A thread's consecutive particles
-    // usually share a cell (the lattice of a cell is ordered with the
-    // azimuthal index innermost), so each thread sums its per-corner
-    // contributions in registers while the cell stays the same and adds them
-    // to the LDS tile once per cell.
-    const int64_t sr = gJ.nx + 1, sm = sr * (gJ.nr + 1), sl = sm * nmod;
-    for (int l = 0; l < 4; l++) {
-        const bool isJ = l < 3;
-        if ((isJ && !doJ) || (!isJ && !doR)) continue;
-        const GridGeom& gg = isJ ? gJ : gR;
-        double* tile_l = tile;
-        C* grid_l = isJ ? a.J + l * sl : a.R;
-        const int bx0 = isJ ? box[0] : box[4], br0 = isJ ? box[2] : box[6];
-        const int TX = isJ ? TXJ : TXR, TR = isJ ? TRJ : TRR;
-        const bool tiled = isJ ? tileJ : tileR;
-        const int64_t nt = isJ ? nJ : nR;
         if (tiled) {
-            for (int64_t i = tid; i < nt; i += DEP_THREADS) tile[i] = 0.0;
-            __syncthreads();
-        }
-        double2 acc[NMOD][4];   // per-cell sums in FP64 in both precisions
-        int cx = -1, cr = 0;
-        // a cell's sums go to the tile, or, for a block without one (its box
-        // too large), to the grid with one atomic per node value and cell
-        auto flush = [&]() __attribute__((always_inline)) {
-            if (cx < 0) return;
-            if (!tiled) {
+            double* tp = tile + c * pns + key + (up ? TX : 0);
 #pragma unroll
-                for (int m = 0; m < NMOD; m++)
+            for (int i = 0; i < PL; i++)
 #pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        R* dst = reinterpret_cast<R*>(grid_l + (cx + (q & 1)) + (int64_t)(cr + (q >> 1)) * sr + m * sm);
-                        unsafeAtomicAdd(dst, (R)acc[m][q].x);
-                        unsafeAtomicAdd(dst + 1, (R)acc[m][q].y);
-                    }
-                return;
-            }
-            const int tx = cx - bx0, tr = cr - br0;
+                for (int k = 0; k < 2; k++) lds_add(tp + i * nn + k, acc[i][k]);
+        } else {
 #pragma unroll
             for (int m = 0; m < NMOD; m++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int t = ((m * TR + (tr + (q >> 1))) * TX + (tx + (q & 1))) * 2;
-                    lds_add(tile_l + t, (double)acc[m][q].x);
-                    lds_add(tile_l + t + 1, (double)acc[m][q].y);
+                for (int k = 0; k < 2; k++) {
+                    R* dst = reinterpret_cast<R*>(grid + (c0 + c) * sl + m * sm + key + k + (up ? sr : 0));
+                    unsafeAtomicAdd(dst, (R)acc[m ? 2 * m - 1 : 0][k]);
+                    // the imaginary part of mode 0 is 0 times the real one
+                    const double im = m ? acc[2 * m][k] : 0.0 * acc[0][k];
+                    if (m || im != 0.0) unsafeAtomicAdd(dst + 1, (R)im);
                 }
-        };
-        for (int h = 0; h < PPT / DEP_G; h++) {
-        double P[3][DEP_G], V[3][DEP_G], Wt[3][DEP_G];   // Wt: row 0 only
-        load_parts(isJ ? a.xh : a.x, P, 3, h);
-        if (isJ) load_parts(a.u, V, 3, h);
-        load_parts(a.w, Wt, 1, h);
-#pragma unroll
-        for (int j = 0; j < DEP_G; j++) {
-            const double wp = Wt[0][j];
-            if (wp == 0.0) continue;
-            double q0;   // weight of this component: w*u_l/gamma for J, w for rho
-            PartGeom pg;
-            if (isJ) {
-                const double u0 = V[0][j], u1 = V[1][j], u2 = V[2][j];
-                if ((fabs(u0) + fabs(u1) + fabs(u2)) == 0.0) continue;
-                if (!part_geom(pg, P[0][j], P[1][j], P[2][j], gg, -1.0)) continue;
-                const double gp = sqrt(1 + u0 * u0 + u1 * u1 + u2 * u2);
-                q0 = (l == 0 ? u0 : l == 1 ? u1 : u2) * wp / gp;
-            } else {
-                if (!part_geom(pg, P[0][j], P[1][j], P[2][j], gg, -1.0)) continue;
-                q0 = wp;
-            }
-            // in-tile test on the cell found here (phase 1 may round differently at a cell edge)
-            const int64_t tx = pg.ix - bx0, tr = pg.ir - br0;
-            if (!tiled || (tx >= 0 && tx + 1 < TX && tr >= 0 && tr + 1 < TR)) {
-                if (pg.ix != cx || pg.ir != cr) {
-                    flush();
-#pragma unroll
-                    for (int m = 0; m < NMOD; m++)
-#pragma unroll
-                        for (int q = 0; q < 4; q++) acc[m][q] = cmk(0.0, 0.0);
-                    cx = (int)pg.ix;
-                    cr = (int)pg.ir;
-                }
-#pragma unroll
-                for (int m = 0; m < NMOD; m++) {
-                    const double2 pv = crs(q0, pg.ph[m]);
-#pragma unroll
-                    for (int q = 0; q < 4; q++)
-                        acc[m][q] = cadd(acc[m][q], crs(pg.S[0][q & 1] * pg.S[1][q >> 1], pv));
-                }
-            } else {
-#pragma unroll
-                for (int m = 0; m < NMOD; m++) {
-                    const double2 pv = crs(q0, pg.ph[m]);
-                    for (int q = 0; q < 4; q++) {
-                        const double2 d = crs(pg.S[0][q & 1] * pg.S[1][q >> 1], pv);
-                        R* dst = reinterpret_cast<R*>(grid_l + (pg.ix + (q & 1)) + (pg.ir + (q >> 1)) * sr + m * sm);
-                        unsafeAtomicAdd(dst, (R)d.x);
-                        unsafeAtomicAdd(dst + 1, (R)d.y);
-                    }
-                }
-            }
         }
-        }
-        flush();
-        if (!tiled) continue;
-        __syncthreads();
-        const bool slot = isJ ? slotJ : slotR;
-        const int64_t n = nt / 2;
-        if (slot) {
-            // tile index (m*TR + rr)*TX + xx -> slot index ((l*nmod + m)*DEP_SLOT_R + rr)*SW + xx
-            // (rho: l = 0 of its own slot array)
-            C* sl_base = isJ ? a.slotJ + (int64_t)blk * (3 * nmod * DEP_SLOT_R * SW) +
-                                   (int64_t)l * nmod * DEP_SLOT_R * SW
-                             : a.slotR + (int64_t)blk * (nmod * DEP_SLOT_R * SW);
-            for (int64_t i = tid; i < n; i += DEP_THREADS) {
-                const int64_t rest = i / TX;
-                sl_base[((rest / TR) * DEP_SLOT_R + rest % TR) * SW + i % TX] =
-                    cmake<R>((R)tile[2 * i], (R)tile[2 * i + 1]);
-            }
-        } else {
-            for (int64_t i = tid; i < n; i += DEP_THREADS) {
-                const R re = (R)tile[2 * i], im = (R)tile[2 * i + 1];
-                if (re == 0 && im == 0) continue;
-                const int64_t xx = i % TX, rest = i / TX, rr = rest % TR, m = rest / TR;
-                R* dst = reinterpret_cast<R*>(grid_l + (bx0 + xx) + (br0 + rr) * sr + m * sm);
-                unsafeAtomicAdd(dst, re);
-                unsafeAtomicAdd(dst + 1, im);
-            }
-        }
-        __syncthreads();   // the tile is zeroed again by the next pass
     }
+}
 
-    const int4 none = make_int4(-1, 0, 0, 0);
-    if (tid == 0) {
-        if (doJ) a.desc[blk] = slotJ ? make_int4(box[2], box[0], TXJ, TRJ) : none;
-        if (doR) a.desc[a.nblocks + blk] = slotR ? make_int4(box[6], box[4], TXR, TRR) : none;
+// ncp components of the tile to the group's slot, or, without one, to the grid;
+// the tile is left zero for the next pass.
+template <int NMOD, typename R>
+__device__ __forceinline__ void dep_writeout(double* tile, int ncp, int pns, int nn, int TX, R* slot, cplx_t<R>* grid,
+                                             int64_t sr, int64_t sm) {
+    typedef R rv2 __attribute__((ext_vector_type(2)));
+    const int n = ncp * pns;
+    if (slot) {
+        for (int i = 2 * threadIdx.x; i < n; i += 2 * DEP_T) {     // pns is even
+            const double2 v = *reinterpret_cast<const double2*>(tile + i);
+            *reinterpret_cast<double2*>(tile + i) = cmk(0.0, 0.0);
+            rv2 t;
+            t[0] = (R)v.x, t[1] = (R)v.y;
+            *reinterpret_cast<rv2*>(slot + i) = t;
+        }
+        return;
     }
+    for (int i = threadIdx.x; i < n; i += DEP_T) {
+        const double v = tile[i];
+        tile[i] = 0.0;
+        if (v == 0.0) continue;      // (the odd value between components among them)
+        const int c = i / pns, at = i - c * pns, k = at / nn, node = at - k * nn, rr = node / TX, xx = node - rr * TX;
+        R* dst = reinterpret_cast<R*>(grid + (int64_t)(c * NMOD + (k + 1) / 2) * sm + xx + rr * sr);
+        unsafeAtomicAdd(dst + (k > 0 && (k & 1) == 0 ? 1 : 0), (R)v);
+        if (k == 0 && 0.0 * v != 0.0) unsafeAtomicAdd(dst + 1, (R)(0.0 * v));    // Im of mode 0: 0 times Re
+    }
+}
+
+// R: precision of momenta, weights and grids (double, or float in mixed
+// precision).  Positions, the push and the cell geometry stay FP64; each
+// corner contribution is formed and summed in FP64, and the LDS tile is FP64
+// in both precisions, rounded to R when it leaves the block.
+template <int NMOD, typename R, int PPL>
+__global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
+    typedef double dvp __attribute__((ext_vector_type(PPL)));
+    constexpr int PL = 2 * NMOD - 1;
+    __shared__ DepWave<PPL> wl[DEP_WAVES];
+    __shared__ __align__(16) double tile[DEP_POOL];
+    __shared__ int red[DEP_WAVES][4];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const GridGeom gJ = frame_geom(a.gJ), gR = frame_geom(a.gR);
+    const int64_t ld = a.ld;
+    const bool doJ = a.J != nullptr, doR = a.R != nullptr;
+    const int64_t sr = gJ.nx + 1, sm = sr * (gJ.nr + 1), sl = sm * NMOD;
+    DepWave<PPL>& L = wl[wv];
+
+    const int grp = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t ib = (int64_t)grp * (DEP_T * PPL) + (int64_t)tid * PPL;
+    double X[3][PPL], H[3][PPL], U[3][PPL], W[PPL];
+    auto load = [&](const auto* p, double (&v)[PPL]) __attribute__((always_inline)) {
+        typedef typename std::remove_cv<typename std::remove_pointer<decltype(p)>::type>::type T;
+        typedef T tvp __attribute__((ext_vector_type(PPL)));
+        if (a.vec && ib + PPL <= a.np) {
+            const tvp t = *reinterpret_cast<const tvp*>(p + ib);
+#pragma unroll
+            for (int k = 0; k < PPL; k++) v[k] = t[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < PPL; k++) v[k] = ib + k < a.np ? (double)p[ib + k] : 0.0;
+        }
+    };
+    // ---- 1. load, push, store, geometry
+    load(a.w, W);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        load(a.x + c * ld, X[c]);
+        load(a.u + c * ld, U[c]);
+    }
+    if (!a.push && doJ) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) load(a.xh + c * ld, H[c]);
+    }
+    for (int i = 2 * tid; i < DEP_POOL; i += 2 * DEP_T) *reinterpret_cast<double2*>(tile + i) = cmk(0.0, 0.0);
+
+    double ig[PPL];      // 1/gamma
+#pragma unroll
+    for (int k = 0; k < PPL; k++) {
+        const double g2 = 1.0 + (U[0][k] * U[0][k] + U[1][k] * U[1][k] + U[2][k] * U[2][k]);
+        double gam;
+        sqrt_rsqrt(g2, gam, ig[k]);
+        if (!(g2 <= 1e300)) ig[k] = 1.0 / sqrt(g2);
+    }
+    if (a.push) {
+        // particle_tools.f90:58-82: x += u*dt/gamma; x_half = (x_old + x_new)/2
+#pragma unroll
+        for (int k = 0; k < PPL; k++) {
+            const double dt_gp = a.dt * ig[k];
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const double xn = X[c][k] + U[c][k] * dt_gp;
+                H[c][k] = 0.5 * (X[c][k] + xn);
+                X[c][k] = xn;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            if (a.vec && ib + PPL <= a.np) {
+                dvp t, h;
+#pragma unroll
+                for (int k = 0; k < PPL; k++) t[k] = X[c][k], h[k] = H[c][k];
+                *reinterpret_cast<dvp*>(a.x + c * ld + ib) = t;
+                *reinterpret_cast<dvp*>(a.xh + c * ld + ib) = h;
+            } else {
+#pragma unroll
+                for (int k = 0; k < PPL; k++)
+                    if (ib + k < a.np) {
+                        a.x[c * ld + ib + k] = X[c][k];
+                        a.xh[c * ld + ib + k] = H[c][k];
+                    }
+            }
+        }
+    }
+    int bx0 = INT_MAX, bx1 = INT_MIN, br0 = INT_MAX, br1 = INT_MIN;
+    int ixJ[PPL], irJ[PPL], ixR[PPL], irR[PPL];
+    bool okJ[PPL], okR[PPL];
+    double2 sR[PPL], pR[PPL];
+#pragma unroll
+    for (int k = 0; k < PPL; k++) {
+        double2 s, p1;
+        okJ[k] = doJ && W[k] != 0.0 && (fabs(U[0][k]) + fabs(U[1][k]) + fabs(U[2][k])) != 0.0 &&
+                 dep_geom(H[0][k], H[1][k], H[2][k], gJ, ixJ[k], irJ[k], s, p1);
+        if (okJ[k]) {
+            bx0 = min(bx0, ixJ[k]), bx1 = max(bx1, ixJ[k]), br0 = min(br0, irJ[k]), br1 = max(br1, irJ[k]);
+            const int o = L.pos(lane * PPL + k);
+            const double wg = W[k] * ig[k];
+            L.s[o] = s;
+            L.p1[o] = p1;
+#pragma unroll
+            for (int c = 0; c < 3; c++) L.q[c][o] = U[c][k] * wg;
+        }
+        okR[k] = doR && W[k] != 0.0 && dep_geom(X[0][k], X[1][k], X[2][k], gR, ixR[k], irR[k], sR[k], pR[k]);
+        if (okR[k]) bx0 = min(bx0, ixR[k]), bx1 = max(bx1, ixR[k]), br0 = min(br0, irR[k]), br1 = max(br1, irR[k]);
+    }
+    bx0 = wave_reduce63<false>(bx0);
+    bx1 = wave_reduce63<true>(bx1);
+    br0 = wave_reduce63<false>(br0);
+    br1 = wave_reduce63<true>(br1);
+    if (lane == 63) {
+        red[wv][0] = bx0, red[wv][1] = bx1, red[wv][2] = br0, red[wv][3] = br1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < DEP_WAVES; i++) {
+        const int b0 = red[i][0], b1 = red[i][1], b2 = red[i][2], b3 = red[i][3];
+        bx0 = i ? min(bx0, b0) : b0;
+        bx1 = i ? max(bx1, b1) : b1;
+        br0 = i ? min(br0, b2) : b2;
+        br1 = i ? max(br1, b3) : b3;
+    }
+    bx0 = __builtin_amdgcn_readfirstlane(bx0);
+    bx1 = __builtin_amdgcn_readfirstlane(bx1);
+    br0 = __builtin_amdgcn_readfirstlane(br0);
+    br1 = __builtin_amdgcn_readfirstlane(br1);
+
+    // ---- 2 and 3
+    int4 d = make_int4(-1, 0, 0, 0);
+    if (bx1 >= bx0) {
+        const int TX = bx1 - bx0 + 2, TR = br1 - br0 + 2;
+        const int64_t nn64 = (int64_t)TX * TR;
+        const int nc = (doJ ? 3 : 0) + (doR ? 1 : 0);
+        const int64_t pns64 = (PL * nn64 + 1) & ~(int64_t)1;        // values per component, even
+        // components per pass; 0: no tile
+        const int per = nc * pns64 <= DEP_POOL ? nc : 3 * pns64 <= DEP_POOL ? 3 : pns64 <= DEP_POOL ? 1 : 0;
+        const bool tiled = per > 0, slotted = tiled && nc * pns64 <= DEP_SLOT;
+        const int nn = tiled ? (int)nn64 : 1, pns = tiled ? (int)pns64 : 0;
+        R* const slot = slotted ? a.slot + (int64_t)grp * DEP_SLOT : nullptr;
+        const int rho0 = doJ ? 3 * pns : 0;         // rho in the slot
+        const int64_t corner = bx0 + br0 * sr;      // grid node of the tile's first node
+        auto keys = [&](const bool (&ok)[PPL], const int (&ix)[PPL], const int (&ir)[PPL], uint32_t (&key)[PPL])
+            __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < PPL; k++)
+                key[k] = !ok[k] ? DEP_SKIP
+                                : tiled ? (uint32_t)((ir[k] - br0) * TX + ix[k] - bx0) : (uint32_t)(ix[k] + ir[k] * sr);
+        };
+        uint32_t key[PPL];
+        if (doJ) {
+            keys(okJ, ixJ, irJ, key);
+            const int nseg = dep_segments<PPL, 3>(L, key);
+            if (per != 1) {
+                dep_pass<NMOD, 3, PPL, R>(L, nseg, 0, tiled, tile, pns, nn, TX, a.J, sr, sm, sl);
+                if (per == 3) {
+                    __syncthreads();
+                    dep_writeout<NMOD, R>(tile, 3, pns, nn, TX, slot, a.J + corner, sr, sm);
+                    __syncthreads();
+                }
+            } else {
+#pragma unroll 1
+                for (int c = 0; c < 3; c++) {
+                    dep_pass<NMOD, 1, PPL, R>(L, nseg, c, true, tile, pns, nn, TX, a.J, sr, sm, sl);
+                    __syncthreads();
+                    dep_writeout<NMOD, R>(tile, 1, pns, nn, TX, slot ? slot + c * pns : nullptr,
+                                          a.J + c * sl + corner, sr, sm);
+                    __syncthreads();
+                }
+            }
+            wave_lds_fence();
+        }
+        if (doR) {
+#pragma unroll
+            for (int k = 0; k < PPL; k++)
+                if (okR[k]) {
+                    const int o = L.pos(lane * PPL + k);
+                    L.s[o] = sR[k];
+                    L.p1[o] = pR[k];
+                    L.q[0][o] = W[k];
+                }
+            keys(okR, ixR, irR, key);
+            const int nseg = dep_segments<PPL, 1>(L, key);
+            dep_pass<NMOD, 1, PPL, R>(L, nseg, 0, tiled, tile + (per == 4 ? rho0 : 0), pns, nn, TX, a.R, sr, sm, sl);
+            if (tiled) {
+                __syncthreads();
+                if (per != 4) {
+                    dep_writeout<NMOD, R>(tile, 1, pns, nn, TX, slot ? slot + rho0 : nullptr, a.R + corner, sr, sm);
+                } else if (slot) {
+                    dep_writeout<NMOD, R>(tile, 4, pns, nn, TX, slot, nullptr, sr, sm);
+                } else {
+                    dep_writeout<NMOD, R>(tile, 3, pns, nn, TX, nullptr, a.J + corner, sr, sm);
+                    dep_writeout<NMOD, R>(tile + rho0, 1, pns, nn, TX, nullptr, a.R + corner, sr, sm);
+                }
+            }
+        }
+        if (slotted) {
+            d = make_int4(br0, bx0, TX, TR);
+            if (a.mask && tid < TR)
+                atomicOr(a.mask + (int64_t)(br0 + tid) * a.words + (grp >> 11), 1u << ((grp >> 6) & 31));
+        }
+    }
+    if (tid == 0) a.desc[grp] = d;
 }
 
 // ------------------------------------------------------------------ slot combine
 //
-// Descriptor d (0 <= d < 2*nblocks; J first, then rho) gets the bucket key
-// which*nrb + first node row (nrb = nr + 1 buckets per grid), or 2*nrb
-// without a slot.
-// A stable radix sort of the keys lists every bucket's slots in block order.
-__global__ void k_slot_keys(const int4* __restrict__ desc, int nb, int nrb, uint32_t* __restrict__ keys) {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    if (d >= 2 * nb) return;
-    const int row = desc[d].x;
-    keys[d] = row >= 0 ? (uint32_t)((d >= nb ? nrb : 0) + row) : (uint32_t)(2 * nrb);
-}
+// One wave per (64 node columns, node row r).  It lists the slots that cover
+// its nodes in group order -- the 64 descriptors of one load and a ballot --
+// and adds their sums to the grids once, so the order of the sum is fixed.
+// The descriptors to look at come from the row's bits of `mask`, or, without
+// one (small launches), are all of them.  (A radix sort of the descriptors by
+// row, which the mask replaced, took a dozen launches and 70 us at 16.7 M
+// particles.)
+constexpr int CMB_T = 256;
 
-// bounds[2*k], bounds[2*k+1]: first and one-past-last sorted position of bucket k (zeroed before)
-__global__ void k_slot_bounds(const uint32_t* __restrict__ keys, int n, uint32_t nkeys, int32_t* __restrict__ bounds) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const uint32_t k = keys[p];
-    if (k >= nkeys) return;
-    if (p == 0 || keys[p - 1] != k) bounds[2 * k] = p;
-    if (p == n - 1 || keys[p + 1] != k) bounds[2 * k + 1] = p + 1;
-}
-
-constexpr int CMB_T = 256, CMB_LIST = 1024;
-
-// One workgroup per (256 node columns, node row r, grid): the slots whose
-// first node row is r - layer (layer < DEP_SLOT_R, their node row `layer` is
-// r) and whose columns overlap the workgroup's are listed in LDS in sorted
-// order (stable compaction with ballots), with their column range; each
-// thread then sums the listed slots that cover its node and adds the sum to
-// the grid once.  The order of the sum is fixed: layer 0 first, blocks in
-// index order within a layer.  The candidates of a layer come from the bucket
-// of row r - layer (sidx and bounds from the sort of the slot keys) or, when
-// bounds is null (small launches, where the sort's dozen launches cost more
-// than the scan), from all nb descriptors in block order: the same slots in
-// the same order, so the two forms give the same sums.
-template <int NMOD, typename RT, int SW>
-__global__ void __launch_bounds__(CMB_T) k_dep_combine(cplx_t<RT>* __restrict__ J, cplx_t<RT>* __restrict__ R,
-                                                        const cplx_t<RT>* __restrict__ slotJ,
-                                                        const cplx_t<RT>* __restrict__ slotR,
-                                                        const int4* __restrict__ desc, const int32_t* __restrict__ sidx,
-                                                        const int32_t* __restrict__ bounds, int nb, int nrb,
-                                                        int64_t sr, int64_t sm, int nx1) {
-    constexpr int NC = 3 * NMOD;
-    const int which = blockIdx.z;
-    typedef cplx_t<RT> C;
-    C* grid = which ? R : J;
-    if (grid == nullptr) return;
-    const C* slot = which ? slotR : slotJ;
-    const int ncomp = which ? NMOD : NC;
-    const int64_t sstride = (int64_t)ncomp * DEP_SLOT_R * SW;
-    const int r = blockIdx.y, xs = blockIdx.x * CMB_T, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int x = xs + tid;
-    __shared__ int4 list[CMB_LIST];   // (4*block + layer, first column, width, 0)
-    __shared__ int wcount[CMB_T / 64];
-    __shared__ int nlist;
-    C acc[NC];
+template <int NMOD, typename RT>
+__global__ void __launch_bounds__(CMB_T) k_dep_combine(DepArgsT<RT> a, int64_t sr, int64_t sm, int nx1) {
+    constexpr int PL = 2 * NMOD - 1;
+    const int r = blockIdx.y, lane = threadIdx.x & 63;
+    const int xs = (blockIdx.x * (CMB_T / 64) + (threadIdx.x >> 6)) * 64, x = xs + lane;
+    if (xs >= nx1) return;
+    const bool doJ = a.J != nullptr, doR = a.R != nullptr;
+    RT acc[4][PL];       // J_x, J_y, J_z, rho
 #pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = cmake<RT>(0, 0);
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int i = 0; i < PL; i++) acc[c][i] = 0;
     bool hit = false;
-    auto drain = [&](int n) __attribute__((always_inline)) {
-        for (int e = 0; e < n; e++) {
-            const int4 ent = list[e];
-            if (x >= ent.y && x < ent.y + ent.z) {
+    auto look = [&](int batch) __attribute__((always_inline)) {
+        const int b = batch * 64 + lane;
+        int4 d = make_int4(-1, 0, 0, 0);
+        if (b < a.ngroups) d = a.desc[b];
+        uint64_t bal = __ballot(d.x >= 0 && r >= d.x && r - d.x < d.w && d.y < xs + 64 && d.y + d.z > xs);
+        while (bal) {
+            const int j = __builtin_ctzll(bal);
+            bal &= bal - 1;
+            const int row = __builtin_amdgcn_readlane(d.x, j), col = __builtin_amdgcn_readlane(d.y, j);
+            const int width = __builtin_amdgcn_readlane(d.z, j), rows = __builtin_amdgcn_readlane(d.w, j);
+            const int nn = width * rows, pns = (PL * nn + 1) & ~1, o = x - col;
+            if (o >= 0 && o < width) {
                 hit = true;
-                const int b = ent.x >> 2, layer = ent.x & 3;
-                const C* sp = slot + (int64_t)b * sstride + layer * SW + (x - ent.y);
+                const RT* sp = a.slot + (int64_t)(batch * 64 + j) * DEP_SLOT + (r - row) * width + o;
+                if (doJ) {
 #pragma unroll
-                for (int c = 0; c < NC; c++)
-                    if (c < ncomp) acc[c] = cadd(acc[c], sp[c * DEP_SLOT_R * SW]);
+                    for (int c = 0; c < 3; c++)
+#pragma unroll
+                        for (int i = 0; i < PL; i++) acc[c][i] += sp[c * pns + i * nn];
+                    sp += 3 * pns;
+                }
+                if (doR) {
+#pragma unroll
+                    for (int i = 0; i < PL; i++) acc[3][i] += sp[i * nn];
+                }
             }
         }
     };
-    if (tid == 0) nlist = 0;
-    __syncthreads();
-    for (int layer = 0; layer < DEP_SLOT_R; layer++) {
-        const int row = r - layer;
-        if (row < 0 || row >= nrb) continue;
-        const int k = which * nrb + row;
-        const int b0 = bounds ? bounds[2 * k] : 0, b1 = bounds ? bounds[2 * k + 1] : nb;
-        for (int q0 = b0; q0 < b1; q0 += CMB_T) {
-            const int q = q0 + tid;
-            int4 ent = make_int4(-1, 0, 0, 0);
-            if (q < b1) {
-                const int b = bounds ? sidx[q] - which * nb : q;
-                const int4 d = desc[which * nb + b];
-                if (d.x == row && layer < d.w && d.y < xs + CMB_T && d.y + d.z > xs)
-                    ent = make_int4(4 * b + layer, d.y, d.z, 0);
-            }
-            // stable compaction: wave ballot + per-wave offsets
-            const unsigned long long m = __ballot(ent.x >= 0);
-            const int before = __popcll(m & ((1ull << lane) - 1ull));
-            if (lane == 0) wcount[wv] = __popcll(m);
-            __syncthreads();
-            int off = nlist;
-            for (int w = 0; w < wv; w++) off += wcount[w];
-            if (ent.x >= 0) list[off + before] = ent;
-            __syncthreads();
-            if (tid == 0) {
-                int tot = 0;
-                for (int w = 0; w < CMB_T / 64; w++) tot += wcount[w];
-                nlist += tot;
-            }
-            __syncthreads();
-            if (nlist > CMB_LIST - CMB_T) {
-                if (x < nx1) drain(nlist);
-                __syncthreads();
-                if (tid == 0) nlist = 0;
-                __syncthreads();
+    if (a.mask) {
+        const uint32_t* mask = a.mask + (int64_t)r * a.words;
+        for (int w0 = 0; w0 < a.words; w0 += 64) {
+            const uint32_t word = w0 + lane < a.words ? mask[w0 + lane] : 0u;
+            uint64_t wb = __ballot(word != 0u);
+            while (wb) {
+                const int j = __builtin_ctzll(wb);
+                wb &= wb - 1;
+                uint32_t bits = (uint32_t)__builtin_amdgcn_readlane((int)word, j);
+                while (bits) {
+                    look((w0 + j) * 32 + __builtin_ctz(bits));
+                    bits &= bits - 1;
+                }
             }
         }
+    } else {
+        for (int i = 0; i * 64 < a.ngroups; i++) look(i);
     }
-    if (x < nx1) drain(nlist);
-    if (x >= nx1 || !hit) return;
-    C* gp = grid + x + (int64_t)r * sr;
+    if (!hit || x >= nx1) return;
+    const int64_t node = x + (int64_t)r * sr;
 #pragma unroll
-    for (int c = 0; c < NC; c++)
-        if (c < ncomp) gp[c * sm] = cadd(gp[c * sm], acc[c]);
+    for (int c = 0; c < 4; c++) {
+        if (c < 3 ? !doJ : !doR) continue;
+        cplx_t<RT>* gp = (c < 3 ? a.J + c * NMOD * sm : a.R) + node;
+#pragma unroll
+        for (int m = 0; m < NMOD; m++) {
+            // the imaginary part of mode 0 is 0 times the real one
+            const cplx_t<RT> v = m ? cmake<RT>(acc[c][2 * m - 1], acc[c][2 * m]) : cmake<RT>(acc[c][0], 0 * acc[c][0]);
+            gp[m * sm] = cadd(gp[m * sm], v);
+        }
+    }
 }
 
 // Stable compaction: flags, exclusive scan, scatter of every particle array.
@@ -890,7 +989,6 @@ static int32_t push_deposit_impl(double* coord, double* coord_half, const R* mom
                                  int32_t np, double dt, double leftX_J, double leftX_rho, const double* Rgrid,
                                  double dx_inv, double dr_inv, double r0, double rmax, int32_t nx, int32_t nr,
                                  int32_t nkO, cplx_t<R>* curr, cplx_t<R>* dens, const double* frame) {
-    typedef cplx_t<R> C;
     CH_TRY(check_resident(np, ld, nkO));
     if (np == 0) return ST_OK;
     DepArgsT<R> a;
@@ -908,81 +1006,44 @@ static int32_t push_deposit_impl(double* coord, double* coord_half, const R* mom
     a.gR.leftX_dev = frame ? frame + 1 : nullptr;
     a.J = curr;
     a.R = dens;
-    {
-        auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 31) == 0; };
-        a.vec4 = (ld % 4 == 0) && al(coord) && al(coord_half) && al(momenta) && al(wghts);
-    }
-    // 512-particle blocks where the particles average 8 or more per cell
-    const bool big = (int64_t)np >= (int64_t)8 * nx * nr;
-    const int ppt = big ? 8 : 4, sw = 8 * ppt;
-    const int nb = (int)blocks_for(np, DEP_THREADS * ppt);
-    const int nmod = nkO + 1, nrb = nr + 1;
-    a.nblocks = nb;
-    a.slotJ = a.J ? static_cast<C*>(scratch(16, (size_t)nb * 3 * nmod * DEP_SLOT_R * sw * sizeof(C))) : nullptr;
-    a.slotR = a.R ? static_cast<C*>(scratch(17, (size_t)nb * nmod * DEP_SLOT_R * sw * sizeof(C))) : nullptr;
-    a.desc = static_cast<int4*>(scratch(18, (size_t)2 * nb * sizeof(int4)));
-    uint32_t* keys = static_cast<uint32_t*>(scratch(19, (size_t)2 * nb * 4 * sizeof(uint32_t)));
-    int32_t* bounds = static_cast<int32_t*>(scratch(23, (size_t)2 * 2 * nrb * sizeof(int32_t)));
-    if ((a.J && !a.slotJ) || (a.R && !a.slotR) || !a.desc || !keys || !bounds) return ST_ENOMEM;
     if (!a.J && !a.R) return ST_OK;
-    KTimer kt(a.J ? KF_DEP_CURR : KF_DEP_DENS);
-    const int64_t sr = nx + 1, sm = sr * (nr + 1);
-    dim3 grid((unsigned)((nx + 1 + CMB_T - 1) / CMB_T), (unsigned)(nr + 1), 2u);
-    // small launches: every combine workgroup scans all descriptors
-    // (DEP_SLOT_R x nb / CMB_T rounds of coalesced L2 reads, 64 B per
-    // descriptor and workgroup) instead of sorting them into buckets, which
-    // takes a dozen dependent launches of about 5 us each; up to 512 blocks
-    // (131072 particles), or while the scans read at most 512 MiB in all (L2
-    // reads: on a 2048 x 256 bunch of 300 k particles, 352 MiB of them take
-    // less time than the sort)
-    const bool scan_all = nb <= 512 || (int64_t)nb * grid.x * grid.y * grid.z <= ((int64_t)1 << 23);
-#define CMB_LAUNCH(N, IDX, BOUNDS)                                                                                \
-    do {                                                                                                          \
-        if (big)                                                                                                  \
-            hipLaunchKernelGGL((k_dep_combine<N, R, 64>), grid, CMB_T, 0, stream(), a.J, a.R, a.slotJ, a.slotR,   \
-                               a.desc, IDX, BOUNDS, nb, nrb, sr, sm, nx + 1);                                     \
-        else                                                                                                      \
-            hipLaunchKernelGGL((k_dep_combine<N, R, 32>), grid, CMB_T, 0, stream(), a.J, a.R, a.slotJ, a.slotR,   \
-                               a.desc, IDX, BOUNDS, nb, nrb, sr, sm, nx + 1);                                     \
-    } while (0)
-    if (scan_all) {
-        // every descriptor of a deposited grid is written by its block
-#define DEP_LAUNCH(N)                                                                                             \
-    do {                                                                                                          \
-        if (big)                                                                                                  \
-            hipLaunchKernelGGL((k_push_deposit<N, R, 8>), nb, DEP_THREADS, 0, stream(), a);                       \
-        else                                                                                                      \
-            hipLaunchKernelGGL((k_push_deposit<N, R, 4>), nb, DEP_THREADS, 0, stream(), a);                       \
-    } while (0)
-        CH_MODE_SWITCH(nkO, DEP_LAUNCH)
-        CH_LAUNCH_CHECK("k_push_deposit");
-#define CMB_SCAN(N) CMB_LAUNCH(N, nullptr, nullptr)
-        CH_MODE_SWITCH(nkO, CMB_SCAN)
-#undef CMB_SCAN
-        CH_LAUNCH_CHECK("k_dep_combine");
-        return ST_OK;
+    if ((int64_t)(nx + 1) * (nr + 1) >= (int64_t)DEP_SKIP)
+        return fail(ST_EUNSUP, "push_deposit: %d x %d nodes per mode", nx + 1, nr + 1);
+    // groups of 512 particles where they average 8 or more per cell and fill
+    // the chip twice over in such groups; else of 256
+    const bool big = (int64_t)np >= (int64_t)8 * nx * nr && np >= 512 * 512;
+    const int ppl = big ? 2 : 1;
+    {
+        auto al = [](const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; };
+        a.vec = ld % ppl == 0 && al(coord, 8 * ppl) && al(coord_half, 8 * ppl) && al(momenta, sizeof(R) * ppl) &&
+                al(wghts, sizeof(R) * ppl);
     }
-    // descriptors of a grid not deposited here read "no slot" (row -1)
-    CH_TRY(fill_bytes(a.desc, 0xFF, (size_t)2 * nb * sizeof(int4)));
+    a.ngroups = (int)blocks_for(np, DEP_T * ppl);
+    // up to 1024 descriptors a combine wave reads them all (16 KiB in L2);
+    // beyond, the deposit marks those of each row
+    const int nbatch = (a.ngroups + 63) / 64;
+    a.words = (nbatch + 31) / 32;
+    const size_t mask_bytes = nbatch > 16 ? (size_t)(nr + 1) * a.words * sizeof(uint32_t) : 0;
+    a.slot = static_cast<R*>(scratch(16, (size_t)a.ngroups * DEP_SLOT * sizeof(R)));
+    a.desc = static_cast<int4*>(scratch(18, (size_t)a.ngroups * sizeof(int4)));
+    a.mask = mask_bytes ? static_cast<uint32_t*>(scratch(19, mask_bytes)) : nullptr;
+    if (!a.slot || !a.desc || (mask_bytes && !a.mask)) return ST_ENOMEM;
+    KTimer kt(a.J ? KF_DEP_CURR : KF_DEP_DENS);
+    if (a.mask) CH_TRY(fill_bytes(a.mask, 0, mask_bytes));
+#define DEP_LAUNCH(N)                                                                       \
+    do {                                                                                    \
+        if (big)                                                                            \
+            hipLaunchKernelGGL((k_push_deposit<N, R, 2>), a.ngroups, DEP_T, 0, stream(), a);      \
+        else                                                                                \
+            hipLaunchKernelGGL((k_push_deposit<N, R, 1>), a.ngroups, DEP_T, 0, stream(), a);      \
+    } while (0)
     CH_MODE_SWITCH(nkO, DEP_LAUNCH)
 #undef DEP_LAUNCH
     CH_LAUNCH_CHECK("k_push_deposit");
-    // bucket the slots by (grid, cell row), in block order
-    const int nd = 2 * nb;
-    uint32_t* keys_tmp = keys + nd;
-    int32_t* idx = reinterpret_cast<int32_t*>(keys + 2 * (size_t)nd);
-    int32_t* idx_tmp = idx + nd;
-    hipLaunchKernelGGL(k_slot_keys, blocks_for(nd, 256), 256, 0, stream(), a.desc, nb, nrb, keys);
-    CH_LAUNCH_CHECK("k_slot_keys");
-    int bits = 1;
-    while ((1u << bits) <= (uint32_t)(2 * nrb)) bits++;
-    CH_TRY(radix_sort_keys(keys, idx, keys_tmp, idx_tmp, nd, bits, 20, 21));
-    CH_TRY(fill_bytes(bounds, 0, (size_t)2 * 2 * nrb * sizeof(int32_t)));
-    hipLaunchKernelGGL(k_slot_bounds, blocks_for(nd, 256), 256, 0, stream(), keys, nd, (uint32_t)(2 * nrb), bounds);
-    CH_LAUNCH_CHECK("k_slot_bounds");
-#define CMB_SORTED(N) CMB_LAUNCH(N, idx, bounds)
-    CH_MODE_SWITCH(nkO, CMB_SORTED)
-#undef CMB_SORTED
+    const int64_t sr = nx + 1, sm = sr * (nr + 1);
+    const dim3 grid((unsigned)((nx + 1 + CMB_T - 1) / CMB_T), (unsigned)(nr + 1));
+#define CMB_LAUNCH(N) hipLaunchKernelGGL((k_dep_combine<N, R>), grid, CMB_T, 0, stream(), a, sr, sm, nx + 1)
+    CH_MODE_SWITCH(nkO, CMB_LAUNCH)
 #undef CMB_LAUNCH
     CH_LAUNCH_CHECK("k_dep_combine");
     return ST_OK;
