@@ -166,6 +166,15 @@ __device__ __forceinline__ void gst2(double2* p, int64_t i, double2 v) {
     ((CH_GLOBAL ch_vd2*)p)[i] = w;
 }
 
+// Workgroups of a 1-D launch go to the 8 XCDs round-robin (workgroup b to XCD
+// b % 8), and each XCD has its own L2.  xcd_block renumbers them so that XCD x
+// takes one contiguous range of the logical block indices: with particles in
+// cell order that is one region of the grid per L2.  A bijection of [0, nb).
+__device__ __forceinline__ int xcd_block(int b, int nb) {
+    const int q = nb >> 3, r = nb & 7, x = b & 7, k = b >> 3;
+    return x * q + (x < r ? x : r) + k;
+}
+
 // ---------------------------------------------------------------- single-precision complex (mixed precision)
 __host__ __device__ inline float2 cmkf(float re, float im) { return make_float2(re, im); }
 __host__ __device__ inline float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }

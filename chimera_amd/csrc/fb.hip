@@ -20,6 +20,7 @@
 #include <complex>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -614,7 +615,7 @@ __device__ __forceinline__ void gemm_epilogue_serial(const FbJobT<R>& J, const F
                                                      const ACC (&acc1)[NI][NACC == 2 ? WN : 1], int Ncol, int n0,
                                                      int x0, int lane, int wr, int wc);
 
-template <typename R, int NACC, int WN, int NI, typename ACC>
+template <typename R, int NACC, int WN, int NI, int EBM = 8, typename ACC>
 __device__ __forceinline__ void gemm_epilogue(const FbJobT<R>& J, const FbGemmArgs& g, const ACC (&acc0)[NI][WN],
                                               const ACC (&acc1)[NI][NACC == 2 ? WN : 1], int Ncol, int n0, int x0,
                                               int lane, int wr, int wc) {
@@ -625,7 +626,8 @@ __device__ __forceinline__ void gemm_epilogue(const FbJobT<R>& J, const FbGemmAr
         return;
     }
     typedef cplx_t<R> C;
-    constexpr int NE = NI * WN * 2, EB0 = gemm_eb((int)sizeof(R), NACC, WN), EB = EB0 < NE ? EB0 : NE;
+    constexpr int NE = NI * WN * 2, EB0 = gemm_eb((int)sizeof(R), NACC, WN), EB1 = EB0 < EBM ? EB0 : EBM;
+    constexpr int EB = EB1 < NE ? EB1 : NE;
     static_assert(NE % EB == 0, "epilogue batch");
     const int nout = J.nout;
     const bool beta = J.beta != 0;
@@ -730,8 +732,9 @@ __device__ __forceinline__ void gemm_epilogue_serial(const FbJobT<R>& J, const F
     }
 }
 
-// Block tile: 64 complex x (128 real rows) x 32*WN columns; 4 waves as 2 x 2,
-// each 64 rows x 16*WN columns.  NACC = 2 keeps a second accumulator set,
+// The tiles of 32 and 16 complex x (GX), for small grids, and any launch that
+// k_fb_gemm_pipe does not take.  Block tile: GX complex x (2*GX real rows) x
+// 32*WN columns; 4 waves as 2 x 2, each GX rows x 16*WN columns.  NACC = 2 keeps a second accumulator set,
 // fed by segment 1 (launch_fb_gemm orders the segments so).  The K-stages of
 // all segments form one pipeline: the global loads of stage t+1 go to
 // registers while the MFMAs of stage t run, then land in the other LDS
@@ -772,8 +775,7 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm(const FbJob* __restri
     const uint32_t ld1 = (uint32_t)((tid % GB_K + S1.ldd * (tid / GB_K)) * (int64_t)sizeof(double));
     const bool plain0 = seg_plain(S0), plain1 = seg_plain(S1);
     auto fetch_seg = [&](const FbSeg& S, int k0, uint32_t la, uint32_t ldo) __attribute__((always_inline)) {
-        // (not in the 128-column FP64 tiles, which have no registers left for it)
-        if (WN < 4 && g.buf_ok && xfull && nfull && k0 + GB_K <= K) {
+        if (g.buf_ok && xfull && nfull && k0 + GB_K <= K) {
             const uint32_t row = (uint32_t)(g.lda * sizeof(double2));
             const __amdgpu_buffer_rsrc_t rs_a = ch_rsrc(S.a0);
 #pragma unroll
@@ -829,8 +831,7 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm(const FbJob* __restri
             const int e = tid + GB_THREADS * i;
             const int xl = e % GX, kk = e / GX;
             const int c = xl & 7, slot = (xl >> 3) * 16 + (c & 3) + 8 * (c >> 2);
-            // (the 128-column tiles always scale: the branch costs them a spill)
-            const double2 v = (WN < 4 && plain) ? ra[i] : seg_finish(S, ra[i], rb[i]);
+            const double2 v = plain ? ra[i] : seg_finish(S, ra[i], rb[i]);
             A[kk * LDA + slot] = v.x;
             A[kk * LDA + slot + 4] = v.y;
         }
@@ -872,7 +873,314 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm(const FbJob* __restri
     gemm_epilogue<double, NACC, WN, NI>(J, g, acc0, acc1, Ncol, n0, x0, lane, wr, wc);
 }
 
-template <int NACC, int WN, int GX = GB_X>
+// ---- tiles of 64 complex x: a software pipeline
+//
+// The same block tile and sums as k_fb_gemm, for launches whose segments are of
+// the two kinds the operators use: A = T(a0), or (A1) A = i T(a0) + s T(a1) with
+// s = +-1.  The loop over the K-stages has no address arithmetic and one
+// barrier: while the MFMAs of stage t run, the values of stage t+1 (loaded
+// during stage t-1) go to the other LDS buffer and the loads of stage t+2 are
+// issued.  FP64 MFMA and FP64 vector work share the SIMD and the chip's power
+// (the clock falls to 2.1 GHz here), so what counts is the work beside the
+// MFMAs.  Measured at 8192 x 512, four modes: grad-div with the Poisson
+// epilogue 3.43 -> 2.87 ms, of which the arithmetic and address work taken out
+// of the loop and the epilogue gave 0.2 ms and the even share of the XCDs 0.2;
+// without staging and epilogue the MFMAs alone take 1.86 ms.  (Tried and
+// dropped: MFMA operands in two register sets, 3.2 ms; three blocks per CU with
+// narrower tiles, 3.0 to 3.2; wave priorities and a staggered start, no gain.)
+//
+// A is kept in LDS as it comes (re, im of x): a row of 2*GB_X values is written
+// as 16-byte vectors, and the lanes read it permuted, row p of a 16-row tile
+// from value 2*(p%4 + 4*(p/8)) + (p/4)%2, so that the (re, im) of one x end in
+// one lane.  Both stages are swizzled instead of padded (A: blocks of 16 values
+// swapped in odd rows; D: k ^ column), which lets three blocks share a CU.
+// Rows past K hold zeros; x past nx and columns past Ncol compute values that
+// the epilogue does not store (x is clamped to the grid, D reads past the
+// matrix return zero by the buffer's bound).
+template <int WN>
+struct GemmPipe {
+    static constexpr int BN = 32 * WN, LDA = 2 * GB_X;
+    static constexpr int A_STAGE = GB_K * LDA, D_STAGE = BN * GB_K;
+    static constexpr int NA = GB_K * GB_X / GB_THREADS, ND = GB_K * BN / GB_THREADS;
+    static constexpr size_t LDS = 2 * (size_t)(A_STAGE + D_STAGE) * sizeof(double);
+    // value v of row k of A, and k of column n of D, in a stage
+    __device__ static int a(int k, int v) { return k * LDA + (v ^ ((k & 1) << 4)); }
+    __device__ static int d(int k, int n) { return n * GB_K + (k ^ (n & 15)); }
+};
+
+// Blocks per CU (waves per SIMD) the registers and the LDS allow.
+constexpr int gemm_pipe_occ(int nacc, int wn) { return nacc * wn >= 2 ? 2 : 3; }
+
+// Buffer of n bytes at p: loads past it return zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ch_rsrc_n(const void* p, uint32_t n) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)n, 0x00020000);
+}
+
+__device__ __forceinline__ void stb_c(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, double2 v) {
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    ch_vd2 w;
+    w.x = v.x, w.y = v.y;
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, w), r, (int)voff, (int)soff, 0);
+}
+
+// Epilogue of a tile wholly inside the output: the same values as
+// gemm_epilogue.  All arrays of an output have its layout, so one lane offset
+// (of its first element) serves them all: rows and columns of the tile go into
+// the instructions' constant and scalar offsets, and no address is computed
+// per element.  EB elements' loads are issued before their stores.
+template <int NACC, int WN, int NI, int EB>
+__device__ __forceinline__ void gemm_epilogue_full(const FbJob& J, const FbGemmArgs& g, const dbl4 (&acc0)[NI][WN],
+                                                   const dbl4 (&acc1)[NI][NACC == 2 ? WN : 1], int n0, int x0, int lane,
+                                                   int wr, int wc) {
+    constexpr int NE = NI * 2;
+    static_assert(NE % EB == 0, "epilogue batch");
+    const int xl = x0 + wr * 8 * NI + (lane >> 4);
+    const uint32_t v0 = (uint32_t)((xl + g.ldo * (n0 + wc * 16 * WN + (lane & 15))) * (int64_t)sizeof(double2));
+    const bool beta = J.beta != 0;
+    const double dti = g.dt_inv;
+    for (int o = 0; o < J.nout; o++) {
+        const FbOut O = J.out[o];
+        const __amdgpu_buffer_rsrc_t rp = ch_rsrc(O.p), rd = ch_rsrc(O.diag), rs = ch_rsrc(O.scale);
+        const __amdgpu_buffer_rsrc_t r1 = ch_rsrc(O.poiss_np1), r0 = ch_rsrc(O.poiss_n), rw = ch_rsrc(O.poiss_w2);
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+            const uint32_t sj = (uint32_t)(16 * j * g.ldo * (int64_t)sizeof(double2));
+#pragma unroll
+            for (int b = 0; b < NE; b += EB) {
+                double2 v[EB], dg[EB], pv[EB], n1[EB], nn[EB];
+                double sc[EB], w2[EB], kx[EB];
+#pragma unroll
+                for (int e = 0; e < EB; e++) {
+                    const int i = (b + e) / 2, h = (b + e) % 2;
+                    const uint32_t ve = v0 + (uint32_t)(8 * i + 4 * h) * 16u;      // a constant offset of the instruction
+                    if (O.diag) {
+                        dg[e] = ldb_c(rd, ve, sj, double2{});
+                        kx[e] = g.kx[xl + 8 * i + 4 * h];
+                    }
+                    if (O.scale) sc[e] = ldb_r(rs, ve / 2, sj / 2, double{});
+                    if (O.poiss) {
+                        n1[e] = ldb_c(r1, ve, sj, double2{});
+                        nn[e] = ldb_c(r0, ve, sj, double2{});
+                        w2[e] = ldb_r(rw, ve / 2, sj / 2, double{});
+                    }
+                    if (O.poiss || beta) pv[e] = ldb_c(rp, ve, sj, double2{});
+                }
+#pragma unroll
+                for (int e = 0; e < EB; e++) {
+                    const int i = (b + e) / 2, h = (b + e) % 2;
+                    v[e] = cmul(O.alpha0, cmk(acc0[i][j][2 * h], acc0[i][j][2 * h + 1]));
+                    if constexpr (NACC == 2) v[e] = cadd(v[e], cmul(O.alpha1, cmk(acc1[i][j][2 * h], acc1[i][j][2 * h + 1])));
+                    if (O.diag) v[e] = cadd(v[e], crs(kx[e], cmul(O.gamma, dg[e])));
+                    if (O.scale) v[e] = crs(sc[e], v[e]);
+                    // maxwell_solvers.f90:153-158: J += (v + (g_np1 - g_n)*dt_inv)*w2_inv
+                    if (O.poiss) v[e] = cadd(pv[e], crs(w2[e], cadd(v[e], crs(dti, csub(n1[e], nn[e])))));
+                    else if (beta) v[e] = cadd(pv[e], v[e]);
+                }
+#pragma unroll
+                for (int e = 0; e < EB; e++) {
+                    const int i = (b + e) / 2, h = (b + e) % 2;
+                    stb_c(rp, v0 + (uint32_t)(8 * i + 4 * h) * 16u, sj, v[e]);
+                }
+            }
+        }
+    }
+}
+
+// KR: some K of the launch is no multiple of GB_K.
+template <int NACC, int WN, bool A1, bool KR>
+__global__ void __launch_bounds__(GB_THREADS, gemm_pipe_occ(NACC, WN)) k_fb_gemm_pipe(const FbJob* __restrict__ jobs,
+                                                                                      FbGemmArgs g, int nx8, int nyt) {
+    typedef GemmPipe<WN> G;
+    constexpr int NI = 4, BN = G::BN, NA = G::NA, ND = G::ND;
+    // every XCD (workgroup id mod 8) takes an eighth of the x tiles, for all jobs
+    // alike; the column tiles of one x tile, which read the same A, are next to
+    // each other there
+    int id = blockIdx.x >> 3;
+    const int yt = id % nyt;
+    id /= nyt;
+    const int n0 = yt * BN, x0 = ((id % nx8) * 8 + (blockIdx.x & 7)) * GB_X;
+    const FbJob& J = jobs[id / nx8];
+    const int Ncol = J.Ncol, K = J.K, nseg = J.nseg;
+    if (n0 >= Ncol || x0 >= g.nx) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave & 1, wc = wave >> 1;
+
+    extern __shared__ __align__(16) double gbp_smem[];
+    double* const As = gbp_smem;                                            // [2][GB_K][LDA]
+    double* const Ds = gbp_smem + 2 * G::A_STAGE;                           // [2][BN][GB_K]
+
+    dbl4 acc0[NI][WN], acc1[NI][NACC == 2 ? WN : 1];
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int j = 0; j < WN; j++) acc0[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+
+    const int sps = (K + GB_K - 1) / GB_K, nst = sps * nseg;
+    const FbSeg S0 = J.seg[0], S1 = J.seg[nseg > 1 ? 1 : 0];
+    const uint32_t row = (uint32_t)(g.lda * sizeof(double2));
+    const uint32_t la0 = seg_lane_a(S0, min(x0 + lane, g.nx - 1), g.nx, g.lda, 0);
+    const uint32_t la1 = seg_lane_a(S1, min(x0 + lane, g.nx - 1), g.nx, g.lda, 0);
+    const uint32_t ldc = (uint32_t)(S0.ldd * sizeof(double));               // bytes per column of D
+    const uint32_t lcol = (uint32_t)(n0 + (tid >> 4)) * ldc + (uint32_t)(tid & 15) * 8u;
+    const uint32_t dbytes = (uint32_t)(Ncol - 1) * ldc + (uint32_t)K * 8u;
+    double2 ra[NA], rb[A1 ? NA : 1];
+    double rd[ND];
+    // loads of stage t: A row k = k0 + wave + 4i of x = x0 + lane; D row k0 + tid%16 of columns n0 + tid/16 + 16i
+    auto fetch = [&](int t) __attribute__((always_inline)) {
+        const bool s = t >= sps;
+        const int k0 = (s ? t - sps : t) * GB_K;
+        const __amdgpu_buffer_rsrc_t rs_a = ch_rsrc(s ? S1.a0 : S0.a0);
+        const uint32_t la = s ? la1 : la0;
+#pragma unroll
+        for (int i = 0; i < NA; i++) ra[i] = ldb_c(rs_a, la, (uint32_t)min(k0 + wave + 4 * i, K - 1) * row, double2{});
+        if constexpr (A1) {
+            const __amdgpu_buffer_rsrc_t rs_b = ch_rsrc(s ? S1.a1 : S0.a1);
+#pragma unroll
+            for (int i = 0; i < NA; i++) rb[i] = ldb_c(rs_b, la, (uint32_t)min(k0 + wave + 4 * i, K - 1) * row, double2{});
+        }
+        const __amdgpu_buffer_rsrc_t rs_d = ch_rsrc_n(s ? S1.D : S0.D, dbytes);
+#pragma unroll
+        for (int i = 0; i < ND; i++) rd[i] = ldb_r(rs_d, lcol, (uint32_t)k0 * 8u + (uint32_t)(16 * i) * ldc, double{});
+    };
+    // the loaded values of stage t to LDS buffer B
+    auto stash = [&](int t, auto B) __attribute__((always_inline)) {
+        const bool s = t >= sps;
+        const int k0 = (s ? t - sps : t) * GB_K;
+        double* const A = As + B.value * G::A_STAGE;
+        double* const D = Ds + B.value * G::D_STAGE;
+        const bool refl = s ? S1.refl : S0.refl;            // T(v) = (-v.x, v.y)
+        if constexpr (A1) {
+            const double sg = s ? S1.c1.x : S0.c1.x;
+            if (refl) {
+#pragma unroll
+                for (int i = 0; i < NA; i++) ra[i] = cmk(fma(-sg, rb[i].x, -ra[i].y), fma(sg, rb[i].y, -ra[i].x));
+            } else {
+#pragma unroll
+                for (int i = 0; i < NA; i++) ra[i] = cmk(fma(sg, rb[i].x, -ra[i].y), fma(sg, rb[i].y, ra[i].x));
+            }
+        } else if (refl) {
+#pragma unroll
+            for (int i = 0; i < NA; i++) ra[i].x = -ra[i].x;
+        }
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+            if (KR && k0 + wave + 4 * i >= K) ra[i] = cmk(0.0, 0.0);
+            *reinterpret_cast<double2*>(A + G::a(wave + 4 * i, 2 * lane)) = ra[i];
+        }
+#pragma unroll
+        for (int i = 0; i < ND; i++) {
+            if (KR && k0 + (tid & 15) >= K) rd[i] = 0.0;
+            D[G::d(tid & 15, (tid >> 4) + 16 * i)] = rd[i];
+        }
+    };
+    const int p16 = lane & 15, kl = lane >> 4;
+    const int arow = G::a(kl, wr * 64 + 2 * ((p16 & 3) + 4 * (p16 >> 3)) + ((p16 >> 2) & 1));
+    // stage t, in LDS buffer B; the preparation of the next ones stands after the
+    // operand reads of quarter SQ
+    constexpr int SQ = A1 || NACC == 2 ? 1 : GB_K / 4 - 1;
+    auto stage = [&](dbl4 (&acc)[NI][WN], int t, auto B) __attribute__((always_inline)) {
+        const double* A = As + B.value * G::A_STAGE;
+        const double* D = Ds + B.value * G::D_STAGE;
+#pragma unroll
+        for (int kq = 0; kq < GB_K / 4; kq++) {
+            double a[NI], b[WN];
+            // (the swizzle swaps the 16-row tiles i, i^1 in odd rows)
+#pragma unroll
+            for (int i = 0; i < NI; i++) a[i] = A[4 * kq * G::LDA + (arow ^ (16 * i))];
+#pragma unroll
+            for (int j = 0; j < WN; j++) b[j] = D[G::d(kl + 4 * kq, wc * 16 * WN + 16 * j + p16)];
+            if (kq == SQ) {
+                stash(t + 1, std::integral_constant<int, 1 - B.value>{});
+                fetch(min(t + 2, nst - 1));
+            }
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int j = 0; j < WN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        __syncthreads();
+    };
+    const std::integral_constant<int, 0> B0;
+    const std::integral_constant<int, 1> B1;
+    // stages [tb, te) into acc; tb even or, for the second segment, of either parity
+    auto run = [&](dbl4 (&acc)[NI][WN], int tb, int te) __attribute__((always_inline)) {
+        int t = tb;
+        if ((t & 1) && t < te) stage(acc, t++, B1);
+        for (; t + 1 < te; t += 2) {
+            stage(acc, t, B0);
+            stage(acc, t + 1, B1);
+        }
+        if (t < te) stage(acc, t, B0);
+    };
+    if (nst > 0) {
+        fetch(0);
+        stash(0, B0);
+        fetch(min(1, nst - 1));
+        __syncthreads();
+        run(acc0, 0, NACC == 2 ? sps : nst);
+    }
+    if constexpr (NACC == 2) {
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+            for (int j = 0; j < WN; j++) acc1[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+        run(acc1, sps, nst);
+    }
+    if (x0 + GB_X <= g.nx && n0 + BN <= Ncol) {
+        constexpr int EB = NACC == 2 ? 4 : 2;
+        gemm_epilogue_full<NACC, WN, NI, EB>(J, g, acc0, acc1, n0, x0, lane, wr, wc);
+    } else {
+        gemm_epilogue_serial<double, NACC, WN, NI>(J, g, acc0, acc1, Ncol, n0, x0, lane, wr, wc);
+    }
+}
+
+// The kind of the segments of a job list: 0: T(a0); 1: i T(a0) + s T(a1), s =
+// +-1; plus 2 where some K is no multiple of GB_K; -1: of neither kind, or too
+// large for 31-bit offsets (k_fb_gemm).
+static int gemm_pipe_kind(const std::vector<FbJob>& jobs, int buf_ok) {
+    int kind = -2, rem = 0;
+    for (const auto& j : jobs) {
+        if (j.K < 1) return -1;
+        rem |= j.K % GB_K != 0;
+        for (int q = 0; q < j.nseg; q++) {
+            const FbSeg& s = j.seg[q];
+            const int k = !s.a1 && s.c0.x == 1.0 && s.c0.y == 0.0 ? 0
+                        : s.a1 && s.c0.x == 0.0 && s.c0.y == 1.0 && fabs(s.c1.x) == 1.0 && s.c1.y == 0.0 ? 1 : -1;
+            if (k < 0 || (kind != -2 && k != kind) || s.ldd != j.seg[0].ldd) return -1;
+            kind = k;
+        }
+    }
+    return buf_ok ? (kind == -2 ? 0 : kind) + 2 * rem : -1;
+}
+
+template <int NACC, int WN, bool A1, bool KR>
+static int32_t launch_gemm_pipe_k(const FbJob* dj, size_t njobs, int maxN, const FbGemmArgs& g) {
+    constexpr size_t lds = GemmPipe<WN>::LDS;
+    static bool attr = false;
+    if (!attr) {
+        CH_HIP(hipFuncSetAttribute((const void*)k_fb_gemm_pipe<NACC, WN, A1, KR>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        attr = true;
+    }
+    const int nx8 = (g.nx + 8 * GB_X - 1) / (8 * GB_X), nyt = (maxN + 32 * WN - 1) / (32 * WN);
+    const unsigned grid = (unsigned)((size_t)nx8 * 8 * nyt * njobs);
+    hipLaunchKernelGGL((k_fb_gemm_pipe<NACC, WN, A1, KR>), grid, GB_THREADS, lds, stream(), dj, g, nx8, nyt);
+    CH_LAUNCH_CHECK("k_fb_gemm_pipe");
+    return ST_OK;
+}
+
+template <int NACC, int WN>
+static int32_t launch_gemm_pipe(const FbJob* dj, size_t njobs, int maxN, const FbGemmArgs& g) {
+    switch (g.pipe) {
+        case 0: return launch_gemm_pipe_k<NACC, WN, false, false>(dj, njobs, maxN, g);
+        case 1: return launch_gemm_pipe_k<NACC, WN, true, false>(dj, njobs, maxN, g);
+        case 2: return launch_gemm_pipe_k<NACC, WN, false, true>(dj, njobs, maxN, g);
+        default: return launch_gemm_pipe_k<NACC, WN, true, true>(dj, njobs, maxN, g);
+    }
+}
+
+template <int NACC, int WN, int GX>
 static int32_t launch_gemm_variant(const FbJob* dj, size_t njobs, int maxN, const FbGemmArgs& g) {
     constexpr int BN = 32 * WN;
     static bool attr = false;
@@ -937,11 +1245,13 @@ static void merge_jobs(std::vector<FbJobT<R>>& two, const std::vector<FbJobT<R>>
 template <typename R>
 static int gemm_offsets_fit(const std::vector<FbJobT<R>>& jobs, const FbGemmArgs& g) {
     const int64_t lim = (int64_t)1 << 31;
-    for (const auto& j : jobs)
+    for (const auto& j : jobs) {
+        if (((int64_t)j.Ncol * g.ldo + g.nx) * (int64_t)sizeof(cplx_t<R>) >= lim) return 0;
         for (int s = 0; s < j.nseg; s++) {
             if (((int64_t)j.K * g.lda + g.nx) * (int64_t)sizeof(cplx_t<R>) >= lim) return 0;
             if (((int64_t)j.K + j.seg[s].ldd * (int64_t)j.Ncol) * (int64_t)sizeof(R) >= lim) return 0;
         }
+    }
     return 1;
 }
 
@@ -972,19 +1282,20 @@ static std::atomic<int> g_mixed_gemm{MIXED_GEMM_BF16X6};
 // One launch of a job table in tile shape `tile` (GT_*) with NACC
 // accumulators; EUNSUP for a shape the form has no kernel for.
 static int32_t gemm_tile_launch(const FbJob* dj, size_t nj, int maxN, const FbGemmArgs& g, int nacc, int tile) {
+    if (tile < GT_H && g.pipe < 0) return ST_EUNSUP;
     if (nacc == 1) {
         switch (tile) {
-            case GT_W4: return launch_gemm_variant<1, 4>(dj, nj, maxN, g);
-            case GT_W2: return launch_gemm_variant<1, 2>(dj, nj, maxN, g);
-            case GT_W1: return launch_gemm_variant<1, 1>(dj, nj, maxN, g);
+            case GT_W4: return launch_gemm_pipe<1, 4>(dj, nj, maxN, g);
+            case GT_W2: return launch_gemm_pipe<1, 2>(dj, nj, maxN, g);
+            case GT_W1: return launch_gemm_pipe<1, 1>(dj, nj, maxN, g);
             case GT_H: return launch_gemm_variant<1, 1, GB_X / 2>(dj, nj, maxN, g);
             default: return launch_gemm_variant<1, 1, GB_X / 4>(dj, nj, maxN, g);
         }
     }
     switch (tile) {
         case GT_W4: return ST_EUNSUP;
-        case GT_W2: return launch_gemm_variant<2, 2>(dj, nj, maxN, g);
-        case GT_W1: return launch_gemm_variant<2, 1>(dj, nj, maxN, g);
+        case GT_W2: return launch_gemm_pipe<2, 2>(dj, nj, maxN, g);
+        case GT_W1: return launch_gemm_pipe<2, 1>(dj, nj, maxN, g);
         case GT_H: return launch_gemm_variant<2, 1, GB_X / 2>(dj, nj, maxN, g);
         default: return launch_gemm_variant<2, 1, GB_X / 4>(dj, nj, maxN, g);
     }
@@ -1146,13 +1457,17 @@ int32_t launch_fb_gemm<double>(const std::vector<FbJob>& jobs, const FbGemmArgs&
         one.clear();
     }
     for (int pass = 0; pass < 2; pass++) {
-        const std::vector<FbJob>& js = pass == 0 ? one : two;
+        std::vector<FbJob>& js = pass == 0 ? one : two;
         if (js.empty()) continue;
+        // the jobs of two segments first, so that the last blocks to start are short
+        std::stable_sort(js.begin(), js.end(), [](const FbJob& a, const FbJob& b) { return a.nseg > b.nseg; });
         int maxN = 0;
         for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
         const FbJob* dj = static_cast<const FbJob*>(device_table(js.data(), js.size() * sizeof(FbJob)));
         if (!dj) return ST_ENOMEM;
-        const int tile = gemm_choose_tile<FbJob>(dj, js, maxN, g, pass + 1, 8);
+        g.pipe = gemm_pipe_kind(js, g.buf_ok);
+        int tile = gemm_choose_tile<FbJob>(dj, js, maxN, g, pass + 1, 8);
+        if (g.pipe < 0 && tile < GT_H) tile = GT_H;
         CH_TRY(gemm_tile_launch(dj, js.size(), maxN, g, pass + 1, tile));
     }
     return ST_OK;

@@ -118,15 +118,6 @@ __device__ __forceinline__ void boris(R u[3], const R f[6], R dt_2) {
     u[2] = Up2 + dt_2 * f[2];
 }
 
-// Workgroups of a 1-D launch go to the 8 XCDs round-robin (workgroup b to XCD
-// b % 8), and each XCD has its own L2.  xcd_block renumbers them so that XCD x
-// takes one contiguous range of the logical block indices: with particles in
-// cell order that is one region of the grid per L2.  A bijection of [0, nb).
-__device__ __forceinline__ int xcd_block(int b, int nb) {
-    const int q = nb >> 3, r = nb & 7, x = b & 7, k = b >> 3;
-    return x * q + (x < r ? x : r) + k;
-}
-
 // ---------------------------------------------------------------- external-field devices
 //
 // The devices of devices.f90 evaluated at a particle, each adding its field to
