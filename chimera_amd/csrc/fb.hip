@@ -25,417 +25,9 @@
 
 #include "common.hpp"
 #include "fb_kernels.hpp"
-#include "fft.hpp"
 #include "../../include/chimera_hip.h"
 
 namespace chimera {
-
-// ================================================================== FFT
-
-const double2* fft_twiddles(int N) {
-    static std::mutex mu;
-    static std::map<int, const double2*> cache;
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = cache.find(N);
-    if (it != cache.end()) return it->second;
-    std::vector<double2> h(N > 0 ? N : 1);
-    for (int k = 0; k < N; k++) {
-        // exact argument reduction: angle = -2 pi k/N, symmetric in k and N-k
-        const long double a = -2.0L * 3.141592653589793238462643383279502884L * (long double)k / (long double)N;
-        h[k] = make_double2((double)cosl(a), (double)sinl(a));
-    }
-    const double2* d = static_cast<const double2*>(shared_table(h.data(), h.size() * sizeof(double2)));
-    if (d) cache[N] = d;
-    return d;
-}
-
-const float2* fft_twiddles_f(int N) {
-    static std::mutex mu;
-    static std::map<int, const float2*> cache;
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = cache.find(N);
-    if (it != cache.end()) return it->second;
-    std::vector<float2> h(N > 0 ? N : 1);
-    for (int k = 0; k < N; k++) {
-        const long double a = -2.0L * 3.141592653589793238462643383279502884L * (long double)k / (long double)N;
-        h[k] = make_float2((float)cosl(a), (float)sinl(a));
-    }
-    const float2* d = static_cast<const float2*>(shared_table(h.data(), h.size() * sizeof(float2)));
-    if (d) cache[N] = d;
-    return d;
-}
-
-// Store of one transformed point: post-multiplier, real scale table, mode
-// normalisation and the ghost row (shared by both line kernels).
-template <typename R>
-__device__ __forceinline__ void fft_store(const FftArgsT<R>& a, int64_t line, int x, cplx_t<R> v) {
-    typedef cplx_t<R> C;
-    const int64_t r = line % a.n_inner, q = line / a.n_inner;
-    if (a.post) v = cmul(v, a.post[x]);
-    if (a.scale) v = crs(a.scale[x + (int64_t)a.N * r], v);
-    int m = 0;
-    if (a.ghost) {
-        m = (int)(q % a.nmodes);
-        if (a.ghost == 2) v = crs((R)(m == 0 ? 0.5 / M_PI : 1.0 / M_PI), v);
-        else if (a.ghost >= 3) v = crs((R)(1.0 / M_PI), v);
-    }
-    C* o = a.out + r * a.out_r + q * a.out_q + x;
-    *o = v;
-    if (a.ghost && r == 0) {
-        // ghost radial row below row 1: zero (fb_io.f90:199), +-row 1 by mode
-        // (grid_deps.f90:248-265), or +row 1 (3) / -row 1 (4) for every mode of
-        // the envelope grid (grid_deps_env.f90:240-283: + when nkO = 0)
-        o[-a.out_r] = a.ghost == 1 ? cmake<R>(0, 0)
-                    : a.ghost == 2 ? (m == 0 ? v : cneg(v))
-                    : a.ghost == 3 ? v : cneg(v);
-    }
-}
-
-template <int EPT, typename R, int TPB = FFT_THREADS>
-__global__ void __launch_bounds__(TPB) k_fft_lines(FftArgsT<R> a) {
-    typedef cplx_t<R> C;
-    constexpr int TOT = EPT * TPB;
-    extern __shared__ __align__(16) unsigned char fft_smem[];
-    C* const sbuf = reinterpret_cast<C*>(fft_smem);
-    const int N = a.N;
-    const int lpb = TOT / N;
-    const int64_t line0 = (int64_t)blockIdx.x * lpb;
-    const C* tw = a.tw;
-    const C* sph = nullptr;
-    if constexpr (EPT == 8) {
-        // lines of up to 2048 points: the loads go to registers first; where
-        // the LDS has room the twiddle table is staged there (the passes read
-        // it there instead of waiting on memory once per pass) and the phase
-        // table formed there while the loads are in flight
-        C vin[EPT];
-#pragma unroll
-        for (int j = 0; j < EPT; j++) {
-            const int i = threadIdx.x + TPB * j;
-            const int64_t line = line0 + i / N;
-            vin[j] = cmake<R>(0, 0);
-            if (line < a.nlines) {
-                const int64_t r = line % a.n_inner, q = line / a.n_inner;
-                vin[j] = a.in[r * a.in_r + q * a.in_q + i % N];
-            }
-        }
-        C* const stw = sbuf + TOT;
-        if (a.tw_lds) {
-            for (int i = threadIdx.x; i < N; i += TPB) stw[i] = a.tw[i];
-            tw = stw;
-        }
-        if (a.ph_at) {
-            // the table of k_phase, formed here: one launch fewer per transform
-            C* const p = stw + N;
-            const double lx = a.ph_leftX_dev ? *a.ph_leftX_dev : a.ph_leftX;
-            for (int i = threadIdx.x; i < N; i += TPB) {
-                double sn, cs;
-                sincos(lx * a.ph_kx[i], &sn, &cs);
-                p[i] = cmake<R>((R)cs, (R)(a.ph_s * sn));
-            }
-            sph = p;
-            __syncthreads();
-        }
-#pragma unroll
-        for (int j = 0; j < EPT; j++) {
-            const int i = threadIdx.x + TPB * j;
-            const int x = i % N;
-            C v = vin[j];
-            if (line0 + i / N < a.nlines) {
-                if (a.pre) v = cmul(v, a.pre[x]);
-                else if (a.ph_at == 1) v = cmul(v, sph[x]);
-            }
-            sbuf[i] = v;
-        }
-    } else {
-        // ---- load (with the per-x pre-multiplier)
-        for (int i = threadIdx.x; i < TOT; i += TPB) {
-            const int64_t line = line0 + i / N;
-            const int x = i % N;
-            C v = cmake<R>(0, 0);
-            if (line < a.nlines) {
-                const int64_t r = line % a.n_inner, q = line / a.n_inner;
-                v = a.in[r * a.in_r + q * a.in_q + x];
-                if (a.pre) v = cmul(v, a.pre[x]);
-            }
-            sbuf[i] = v;
-        }
-    }
-    __syncthreads();
-    fft_lds<EPT, R, TPB>(sbuf, N, a.log2N, a.sign, tw);
-    if (a.filtr) {
-        // fb_io.f90:263: multiply the first nxfilt points, transform back
-        for (int i = threadIdx.x; i < TOT; i += TPB) {
-            const int x = i % N;
-            if (x < a.nxfilt) sbuf[i] = crs(a.filtr[x], sbuf[i]);
-        }
-        __syncthreads();
-        fft_lds<EPT, R, TPB>(sbuf, N, a.log2N, -a.sign, tw);
-    }
-    // ---- store (with post-multiplier, real scale table, mode normalisation)
-    for (int i = threadIdx.x; i < TOT; i += TPB) {
-        const int64_t line = line0 + i / N;
-        if (line >= a.nlines) continue;
-        const int x = i % N;
-        C v = sbuf[i];
-        if (a.ph_at == 2) v = cmul(v, sph[x]);
-        fft_store<R>(a, line, x, v);
-    }
-}
-
-// ---- lengths that are not powers of two (Bluestein)
-// A length-N DFT of sign s is X_k = c_k * sum_n (x_n c_n) conj(c_(k-n)) with the
-// chirp c_n = exp(s i pi n^2 / N) (from nk = (n^2 + k^2 - (k-n)^2) / 2): a
-// circular convolution, of power-of-two length L >= 2N - 1, of the chirped,
-// zero-padded line with g, g[m] = conj(c_|m|) for |m| < N.  ghat = FFT_L(g) / L,
-// so that IFFT_L(FFT_L(a) * ghat) (both unnormalised) is the convolution.  The
-// tables are built in long double with the angle pi (n^2 mod 2N) / N reduced
-// exactly, then rounded to R.
-static void host_fft_ld(std::vector<std::complex<long double>>& v) {
-    // iterative radix-2, forward (exp(-2 pi i jk / L)), in place
-    const size_t L = v.size();
-    for (size_t i = 1, j = 0; i < L; i++) {
-        size_t bit = L >> 1;
-        for (; j & bit; bit >>= 1) j ^= bit;
-        j ^= bit;
-        if (i < j) std::swap(v[i], v[j]);
-    }
-    const long double pi = 3.141592653589793238462643383279502884L;
-    for (size_t len = 2; len <= L; len <<= 1) {
-        for (size_t i = 0; i < L; i += len) {
-            for (size_t k = 0; k < len / 2; k++) {
-                const long double ang = -2.0L * pi * (long double)k / (long double)len;
-                const std::complex<long double> w(cosl(ang), sinl(ang));
-                const std::complex<long double> u = v[i + k], t = w * v[i + k + len / 2];
-                v[i + k] = u + t;
-                v[i + k + len / 2] = u - t;
-            }
-        }
-    }
-}
-
-int bluestein_length(int N) {
-    int L = 1;
-    while (L < 2 * N - 1) L <<= 1;
-    return L;
-}
-
-template <typename R>
-static int32_t bluestein_tables(int N, int sign, const cplx_t<R>** chirp, const cplx_t<R>** ghat) {
-    typedef cplx_t<R> C;
-    static std::mutex mu;
-    static std::map<std::pair<int, int>, std::pair<const C*, const C*>> cache;
-    std::lock_guard<std::mutex> lk(mu);
-    const auto key = std::make_pair(N, sign);
-    auto it = cache.find(key);
-    if (it == cache.end()) {
-        const int L = bluestein_length(N);
-        const long double pi = 3.141592653589793238462643383279502884L;
-        std::vector<std::complex<long double>> c(N), g(L, std::complex<long double>(0, 0));
-        for (int n = 0; n < N; n++) {
-            const long long n2 = ((long long)n * n) % (2LL * N);
-            const long double ang = (long double)sign * pi * (long double)n2 / (long double)N;
-            c[n] = std::complex<long double>(cosl(ang), sinl(ang));
-        }
-        g[0] = std::conj(c[0]);
-        for (int m = 1; m < N; m++) g[m] = g[L - m] = std::conj(c[m]);
-        host_fft_ld(g);
-        std::vector<C> hc(N), hg(L);
-        for (int n = 0; n < N; n++) hc[n] = cmake<R>((R)c[n].real(), (R)c[n].imag());
-        for (int k = 0; k < L; k++) hg[k] = cmake<R>((R)(g[k].real() / L), (R)(g[k].imag() / L));
-        const C* dc = static_cast<const C*>(shared_table(hc.data(), hc.size() * sizeof(C)));
-        const C* dg = static_cast<const C*>(shared_table(hg.data(), hg.size() * sizeof(C)));
-        if (!dc || !dg) return ST_ENOMEM;
-        it = cache.emplace(key, std::make_pair(dc, dg)).first;
-    }
-    *chirp = it->second.first;
-    *ghat = it->second.second;
-    return ST_OK;
-}
-
-// The convolution step on the lines of buf (stride L): forward FFT, times ghat,
-// unnormalised backward FFT.
-template <int EPT, typename R>
-__device__ __forceinline__ void bluestein_conv(cplx_t<R>* buf, int L, int log2L, const cplx_t<R>* __restrict__ ghat,
-                                               const cplx_t<R>* __restrict__ tw) {
-    constexpr int TOT = EPT * FFT_THREADS;
-    fft_lds<EPT, R>(buf, L, log2L, -1, tw);
-    for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) buf[i] = cmul(buf[i], ghat[i & (L - 1)]);
-    __syncthreads();
-    fft_lds<EPT, R>(buf, L, log2L, +1, tw);
-}
-
-// Lines of length N (not a power of two, 2N - 1 <= 8192) through Bluestein:
-// TOT / L lines per block, each in L points of LDS.  Same loads, pre/post
-// multipliers, absorbing-layer pass and stores as k_fft_lines.
-template <int EPT, typename R>
-__global__ void __launch_bounds__(FFT_THREADS) k_fft_bluestein(FftArgsT<R> a) {
-    typedef cplx_t<R> C;
-    constexpr int TOT = EPT * FFT_THREADS;
-    extern __shared__ __align__(16) unsigned char fft_smem[];
-    C* const sbuf = reinterpret_cast<C*>(fft_smem);
-    const int N = a.N, lm = a.L - 1;
-    const int64_t line0 = (int64_t)blockIdx.x * (TOT >> a.log2L);
-    for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
-        const int64_t line = line0 + (i >> a.log2L);
-        const int x = i & lm;
-        C v = cmake<R>(0, 0);
-        if (x < N && line < a.nlines) {
-            const int64_t r = line % a.n_inner, q = line / a.n_inner;
-            v = a.in[r * a.in_r + q * a.in_q + x];
-            if (a.pre) v = cmul(v, a.pre[x]);
-            v = cmul(v, a.bs_chirp[x]);
-        }
-        sbuf[i] = v;
-    }
-    __syncthreads();
-    bluestein_conv<EPT, R>(sbuf, a.L, a.log2L, a.bs_ghat, a.tw);
-    const C* chirp = a.bs_chirp;
-    if (a.filtr) {
-        // fb_io.f90:263: multiply the first nxfilt points, transform back
-        for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
-            const int x = i & lm;
-            C v = cmake<R>(0, 0);
-            if (x < N) {
-                v = cmul(sbuf[i], a.bs_chirp[x]);
-                if (x < a.nxfilt) v = crs(a.filtr[x], v);
-                v = cmul(v, a.bs_chirp2[x]);
-            }
-            sbuf[i] = v;
-        }
-        __syncthreads();
-        bluestein_conv<EPT, R>(sbuf, a.L, a.log2L, a.bs_ghat2, a.tw);
-        chirp = a.bs_chirp2;
-    }
-    for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
-        const int64_t line = line0 + (i >> a.log2L);
-        const int x = i & lm;
-        if (x >= N || line >= a.nlines) continue;
-        fft_store<R>(a, line, x, cmul(sbuf[i], chirp[x]));
-    }
-}
-
-int32_t fft_length_check(int N) {
-    if (N < 1 || N > 8192 || ((N & (N - 1)) != 0 && bluestein_length(N) > 8192))
-        return fail(ST_EUNSUP,
-                    "FFT length %d: this build transforms powers of two up to 8192 and other lengths up to 4096 "
-                    "along x", N);
-    return ST_OK;
-}
-
-template <typename R>
-static int32_t launch_fft_bluestein(FftArgsT<R> a) {
-    typedef cplx_t<R> C;
-    const int N = a.N, L = bluestein_length(N);
-    a.L = L;
-    a.log2L = 0;
-    while ((1 << a.log2L) < L) a.log2L++;
-    if constexpr (sizeof(R) == 8) a.tw = fft_twiddles(L);
-    else a.tw = fft_twiddles_f(L);
-    if (!a.tw) return ST_ENOMEM;
-    CH_TRY(bluestein_tables<R>(N, a.sign, &a.bs_chirp, &a.bs_ghat));
-    if (a.filtr) CH_TRY(bluestein_tables<R>(N, -a.sign, &a.bs_chirp2, &a.bs_ghat2));
-    a.tw_lds = 0;
-    if (a.ph_at) {
-        CH_TRY(make_phase<R>(a.ph_table, a.ph_kx, a.ph_leftX, a.ph_s, N, a.ph_leftX_dev));
-        if (a.ph_at == 1) a.pre = a.ph_table;
-        else a.post = a.ph_table;
-        a.ph_at = 0;
-    }
-    const int ept = L <= 2048 ? 8 : L / FFT_THREADS;
-    const int tot = ept * FFT_THREADS;
-    const unsigned grid = (unsigned)((a.nlines + tot / L - 1) / (tot / L));
-    const size_t shmem = (size_t)tot * sizeof(C);
-    static bool attr_done = false;
-    if (!attr_done) {
-        CH_HIP(hipFuncSetAttribute((const void*)k_fft_bluestein<8, R>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(8 * FFT_THREADS * sizeof(C))));
-        CH_HIP(hipFuncSetAttribute((const void*)k_fft_bluestein<16, R>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(16 * FFT_THREADS * sizeof(C))));
-        CH_HIP(hipFuncSetAttribute((const void*)k_fft_bluestein<32, R>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(32 * FFT_THREADS * sizeof(C))));
-        attr_done = true;
-    }
-    KTimer kt(KF_FFT);
-    switch (ept) {
-        case 8:
-            hipLaunchKernelGGL((k_fft_bluestein<8, R>), grid, FFT_THREADS, shmem, stream(), a);
-            break;
-        case 16:
-            hipLaunchKernelGGL((k_fft_bluestein<16, R>), grid, FFT_THREADS, shmem, stream(), a);
-            break;
-        case 32:
-            hipLaunchKernelGGL((k_fft_bluestein<32, R>), grid, FFT_THREADS, shmem, stream(), a);
-            break;
-        default:
-            return fail(ST_EUNSUP, "FFT length %d", N);
-    }
-    CH_LAUNCH_CHECK("k_fft_bluestein");
-    return ST_OK;
-}
-
-// Threads per workgroup for lines of 4096 and 8192 points, 8 points each.
-constexpr int FFT_4K_TPB = 4096 / 8, FFT_8K_TPB = 8192 / 8;
-
-template <typename R>
-int32_t launch_fft(FftArgsT<R> a) {
-    typedef cplx_t<R> C;
-    if (a.nlines <= 0) return ST_OK;
-    const int N = a.N;
-    CH_TRY(fft_length_check(N));
-    if ((N & (N - 1)) != 0) return launch_fft_bluestein<R>(a);
-    int l2 = 0;
-    while ((1 << l2) < N) l2++;
-    a.log2N = l2;
-    if constexpr (sizeof(R) == 8) a.tw = fft_twiddles(N);
-    else a.tw = fft_twiddles_f(N);
-    if (!a.tw) return ST_ENOMEM;
-    // every line length runs 8 points a thread (radix-8 passes): lines of up
-    // to 2048 points with 256 threads, several lines per workgroup; longer
-    // lines fill a workgroup's LDS alone (64 and 128 KiB in complex128) with
-    // N / 8 threads, 8 and 16 waves, to hide the passes' LDS latency
-    const int tpb = N <= 2048 ? FFT_THREADS : N / 8;
-    const int ept = 8;
-    const int tot = ept * tpb;
-    const int lpb = tot / N;
-    const unsigned grid = (unsigned)((a.nlines + lpb - 1) / lpb);
-    // LDS of an EPT = 8 workgroup kept within 48 KiB (three per CU): the
-    // twiddles and the phase table are staged there only when they fit
-    a.tw_lds = ept == 8 && (size_t)(tot + N) * sizeof(C) <= 48 * 1024;
-    if (a.ph_at && !(a.tw_lds && (size_t)(tot + 2 * N) * sizeof(C) <= 48 * 1024)) {
-        // no LDS room for the phase table in the transform: k_phase forms it
-        CH_TRY(make_phase<R>(a.ph_table, a.ph_kx, a.ph_leftX, a.ph_s, N, a.ph_leftX_dev));
-        if (a.ph_at == 1) a.pre = a.ph_table;
-        else a.post = a.ph_table;
-        a.ph_at = 0;
-    }
-    const size_t shmem = (size_t)(tot + (a.tw_lds ? N : 0) + (a.ph_at ? N : 0)) * sizeof(C);
-    static bool attr_done = false;
-    if (!attr_done) {
-        // complex128 lines of 4096 and 8192 points use 64 and 128 KiB of LDS per
-        // workgroup; EPT = 8 at most 64 KiB (2048 complex128 points and their twiddles)
-        CH_HIP(hipFuncSetAttribute((const void*)k_fft_lines<8, R>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(64 * 1024)));
-        CH_HIP(hipFuncSetAttribute((const void*)k_fft_lines<8, R, FFT_4K_TPB>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(4096 * sizeof(C))));
-        CH_HIP(hipFuncSetAttribute((const void*)k_fft_lines<8, R, FFT_8K_TPB>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(8192 * sizeof(C))));
-        attr_done = true;
-    }
-    KTimer kt(KF_FFT);
-    if (tpb == FFT_THREADS) {
-        hipLaunchKernelGGL((k_fft_lines<8, R>), grid, FFT_THREADS, shmem, stream(), a);
-    } else if (tpb == FFT_4K_TPB) {
-        hipLaunchKernelGGL((k_fft_lines<8, R, FFT_4K_TPB>), grid, FFT_4K_TPB, shmem, stream(), a);
-    } else if (tpb == FFT_8K_TPB) {
-        hipLaunchKernelGGL((k_fft_lines<8, R, FFT_8K_TPB>), grid, FFT_8K_TPB, shmem, stream(), a);
-    } else {
-        return fail(ST_EUNSUP, "FFT length %d", N);
-    }
-    CH_LAUNCH_CHECK("k_fft_lines");
-    return ST_OK;
-}
-template int32_t launch_fft<double>(FftArgsT<double>);
-template int32_t launch_fft<float>(FftArgsT<float>);
 
 // Per-x phase exp(s*i*kx*leftX) (fb_io.f90:40, :120, :202), on the device.
 template <typename R>

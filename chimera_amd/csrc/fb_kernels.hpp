@@ -28,19 +28,16 @@ struct FftArgsT {
                            // 3, 4: eb_correction_env (1/pi, +row 1 / -row 1)
     int nmodes;            // mode = q % nmodes (ghost != 0)
     int sign;              // -1 FFTW_FORWARD, +1 FFTW_BACKWARD
-    int N, log2N;
-    const C* tw;
+    int N;
+    const C* tw;           // set by launch_fft
     // per-x phase exp(ph_s*i*kx*leftX) (leftX from ph_leftX_dev when set) as
     // the pre (ph_at = 1) or post (ph_at = 2) multiplier: formed inside the
-    // kernel for lines of up to 2048 points when its LDS has room, else by
-    // k_phase into ph_table
+    // kernel for up to FFT_PHASE_POINTS points, else by k_phase into ph_table
     int ph_at;
-    int tw_lds;            // set by launch_fft: twiddle table staged in LDS (EPT = 8)
     // set by launch_fft when N is not a power of two: the line is transformed
     // as a circular convolution of power-of-two length L >= 2N-1 (Bluestein),
     // bs_chirp/bs_ghat for the transform of sign `sign`, bs_chirp2/bs_ghat2 for
     // the transform back of fb_filtr (sign -sign)
-    int L, log2L;
     const C* bs_chirp;
     const C* bs_ghat;
     const C* bs_chirp2;

@@ -1,183 +1,250 @@
-// fft.hpp -- batched complex FFT along x (R = double: complex128, R = float:
-// complex64), one block of TPB threads (256 by default) per TOT = TPB*EPT
-// points of LDS (one line of length N = TOT, or TOT/N lines).
+// fft.hpp -- complex FFT of one line of N = 2^n points, n <= 13, in the registers
+// of T = N/E threads (R = double: complex128, R = float: complex64).
 //
-// Stockham autosort formulation: every pass reads R points at stride N/R,
-// twiddles them, does a radix-R DFT and writes them back in natural order, so
-// no bit reversal is needed.  All points of a pass are held in registers
-// between one barrier and the next, so a single LDS buffer suffices and a line
-// of 8192 points (128 KiB) fits in one workgroup.  Radix 8 (with one radix-4 or
-// radix-2 pass last) when a thread holds a multiple of eight points, else radix
-// 4 with one radix-2 pass first when log2 N is odd.  Twiddles come from a table tw[k] =
-// exp(-2 pi i k/N) built on the host in long double and rounded to R.  Sign conventions are
-// FFTW's: FORWARD = exp(-2 pi i jk/N), BACKWARD = exp(+...), both unnormalised.
+// Stockham autosort formulation.  Thread t holds the points x = t + T*e, e < E,
+// before and after the transform.  A pass of radix Q takes Q points at stride
+// N/Q, which are the thread's own (e = q + r*E/Q, r < Q, for its E/Q
+// butterflies q), twiddles them, does a Q-point DFT in registers and puts the
+// results in natural order.  Only between two passes do the points change
+// threads, through LDS: two exchanges for the three passes of 512 points and
+// more, one from 64, none below (a thread does the whole line).  Lines of up to
+// 1024 points stay within one wave, whose exchanges need no barrier.
+//
+// The exchanges pad one value after every 16, which puts the strided stores of
+// the first passes (stride 16 or 32) on distinct banks.  Complex128 lines and
+// complex64 lines of 8192 points exchange the real and the imaginary parts one
+// after the other, so that two or three lines of 8192 points share a CU
+// (complex64, 6144 lines: 380 us with one exchange of both parts and two lines
+// on a CU, 305 us so).
+//
+// Twiddles are read from a table built on the host in long double and rounded
+// to R, stored in the order in which the threads read it (coalesced): for each
+// pass after the first, W^(k r N/(Ns Q)) at [r - 1][k], W = exp(-2 pi i/N).  Only
+// the forward transform (FFTW's sign, exp(-2 pi i jk/N)) is coded; the backward
+// one conjugates before and after.  Both are unnormalised.
 #pragma once
 
 #include "common.hpp"
 
 namespace chimera {
 
-constexpr int FFT_THREADS = 256;
+// Points per thread and the radices of the passes, by N.
+template <int N> struct FftPlan { static constexpr int E = N, R0 = N, R1 = 1, R2 = 1; };     // N <= 32: one thread
+template <> struct FftPlan<64> { static constexpr int E = 8, R0 = 8, R1 = 8, R2 = 1; };
+template <> struct FftPlan<128> { static constexpr int E = 16, R0 = 16, R1 = 8, R2 = 1; };
+template <> struct FftPlan<256> { static constexpr int E = 16, R0 = 16, R1 = 16, R2 = 1; };
+template <> struct FftPlan<512> { static constexpr int E = 8, R0 = 8, R1 = 8, R2 = 8; };
+template <> struct FftPlan<1024> { static constexpr int E = 16, R0 = 16, R1 = 8, R2 = 8; };
+template <> struct FftPlan<2048> { static constexpr int E = 16, R0 = 16, R1 = 16, R2 = 8; };
+template <> struct FftPlan<4096> { static constexpr int E = 16, R0 = 16, R1 = 16, R2 = 16; };
+template <> struct FftPlan<8192> { static constexpr int E = 32, R0 = 32, R1 = 16, R2 = 16; };
 
+// Whether real and imaginary parts are exchanged one after the other.
+template <int N, typename C>
+constexpr bool fft_parts() { return sizeof(C) == 16 || N == 8192; }
+
+// Block shape of the line kernels: one line of T > 64 threads, or 64 / T lines in one wave.
+template <int N, typename R>
+struct FftShape {
+    static constexpr int E = FftPlan<N>::E, T = N / E, TPB = T > 64 ? T : 64, LINES = TPB / T;
+    static constexpr size_t LS = (N + N / 16) * (fft_parts<N, cplx_t<R>>() ? 1 : 2) * sizeof(R);    // LDS bytes of a line
+    static constexpr size_t LDS = T > 1 ? LINES * LS : 0;
+};
+
+template <typename C> __device__ __forceinline__ C cmi(C a) { C r; r.x = a.y, r.y = -a.x; return r; }    // -i a
+
+// Forward DFTs of Q points in registers, natural order in and out.
+template <int Q, typename C>
+struct Dft;
 template <typename C>
-__device__ __forceinline__ C tw_get(const C* __restrict__ tw, int idx, int sign) {
-    const C w = tw[idx];
-    return sign < 0 ? w : cconj(w);
+struct Dft<1, C> { __device__ static __forceinline__ void go(C*) {} };
+template <typename C>
+struct Dft<2, C> {
+    __device__ static __forceinline__ void go(C* v) {
+        const C a = v[0], b = v[1];
+        v[0] = cadd(a, b);
+        v[1] = csub(a, b);
+    }
+};
+template <typename C>
+struct Dft<4, C> {
+    __device__ static __forceinline__ void go(C* v) {
+        const C s0 = cadd(v[0], v[2]), d0 = csub(v[0], v[2]), s1 = cadd(v[1], v[3]), d1 = cmi(csub(v[1], v[3]));
+        v[0] = cadd(s0, s1);
+        v[1] = cadd(d0, d1);
+        v[2] = csub(s0, s1);
+        v[3] = csub(d0, d1);
+    }
+};
+
+// exp(-2 pi i k/32)
+__device__ __forceinline__ constexpr double w32_cos(int k) {
+    constexpr double c[9] = {1.0, 0.98078528040323044913, 0.92387953251128675613, 0.83146961230254523708,
+                             0.70710678118654752440, 0.55557023301960222474, 0.38268343236508977173,
+                             0.19509032201612826785, 0.0};
+    k &= 31;
+    return k <= 8 ? c[k] : k <= 16 ? -c[16 - k] : k <= 24 ? -c[k - 16] : c[32 - k];
+}
+// v times exp(-2 pi i k/32), k a constant
+template <int K, typename C>
+__device__ __forceinline__ C w32(C v) {
+    typedef decltype(v.x) R;
+    constexpr int k = K & 31;
+    if constexpr (k == 0) return v;
+    else if constexpr (k == 8) return cmi(v);
+    else if constexpr (k == 4) {
+        C r = cadd(v, cmi(v));
+        r.x *= (R)0.70710678118654752440, r.y *= (R)0.70710678118654752440;
+        return r;
+    } else if constexpr (k == 12) {
+        C r = csub(cmi(v), v);
+        r.x *= (R)0.70710678118654752440, r.y *= (R)0.70710678118654752440;
+        return r;
+    } else {
+        constexpr double c = w32_cos(k), s = -w32_cos(k - 8);       // sin of -2 pi k/32
+        C w;
+        w.x = (R)c, w.y = (R)s;
+        return cmul(v, w);
+    }
 }
 
-template <int EPT, typename R, int TPB = FFT_THREADS>
-__device__ __forceinline__ void fft_pass_r4(cplx_t<R>* buf, int N, int Ns, int sign, const cplx_t<R>* __restrict__ tw) {
-    typedef cplx_t<R> C;
-    constexpr int NB = EPT / 4;
-    const int tid = threadIdx.x;
-    const int q4 = N >> 2;
-    C v[NB][4];
-#pragma unroll
-    for (int q = 0; q < NB; q++) {
-        const int b = tid + TPB * q;
-        const int line = b / q4, j = b - line * q4;
-        const C* src = buf + line * N + j;
-#pragma unroll
-        for (int r = 0; r < 4; r++) v[q][r] = src[r * q4];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < NB; q++) {
-        const int b = tid + TPB * q;
-        const int line = b / q4, j = b - line * q4;
-        const int k = j % Ns;
-        if (Ns > 1) {
-            const int step = N / (Ns * 4);
-#pragma unroll
-            for (int r = 1; r < 4; r++) v[q][r] = cmul(v[q][r], tw_get(tw, k * r * step, sign));
+// Q = P * S points: S-strided P-point DFTs, twiddles, S-point DFTs (S = 2 or 4).
+template <int P, int S, int J, int K, typename C>
+__device__ __forceinline__ void dft_twiddle(C (&y)[S][P]) {
+    if constexpr (J < S) {
+        if constexpr (K < P) {
+            y[J][K] = w32<J * K * 32 / (P * S)>(y[J][K]);
+            dft_twiddle<P, S, J, K + 1>(y);
+        } else {
+            dft_twiddle<P, S, J + 1, 0>(y);
         }
-        const C a0 = cadd(v[q][0], v[q][2]), a1 = csub(v[q][0], v[q][2]);
-        const C a2 = cadd(v[q][1], v[q][3]);
-        C a3 = csub(v[q][1], v[q][3]);
-        a3 = sign < 0 ? cmake<R>(a3.y, -a3.x) : cmake<R>(-a3.y, a3.x);  // times -i (forward) or +i
-        C* dst = buf + line * N + (j / Ns) * Ns * 4 + k;
-        dst[0] = cadd(a0, a2);
-        dst[Ns] = cadd(a1, a3);
-        dst[2 * Ns] = csub(a0, a2);
-        dst[3 * Ns] = csub(a1, a3);
     }
-    __syncthreads();
 }
-
-template <int EPT, typename R, int TPB = FFT_THREADS>
-__device__ __forceinline__ void fft_pass_r2(cplx_t<R>* buf, int N, int Ns, int sign, const cplx_t<R>* __restrict__ tw) {
-    typedef cplx_t<R> C;
-    constexpr int NB = EPT / 2;
-    const int tid = threadIdx.x;
-    const int q2 = N >> 1;
-    C v[NB][2];
+template <int P, int S, typename C>
+__device__ __forceinline__ void dft_split(C* v) {
+    C y[S][P];
 #pragma unroll
-    for (int q = 0; q < NB; q++) {
-        const int b = tid + TPB * q;
-        const int line = b / q2, j = b - line * q2;
-        v[q][0] = buf[line * N + j];
-        v[q][1] = buf[line * N + j + q2];
-    }
-    __syncthreads();
+    for (int j = 0; j < S; j++) {
 #pragma unroll
-    for (int q = 0; q < NB; q++) {
-        const int b = tid + TPB * q;
-        const int line = b / q2, j = b - line * q2;
-        const int k = j % Ns;
-        if (Ns > 1) v[q][1] = cmul(v[q][1], tw_get(tw, k * (N / (Ns * 2)), sign));
-        C* dst = buf + line * N + (j / Ns) * Ns * 2 + k;
-        dst[0] = cadd(v[q][0], v[q][1]);
-        dst[Ns] = csub(v[q][0], v[q][1]);
+        for (int n = 0; n < P; n++) y[j][n] = v[S * n + j];
+        Dft<P, C>::go(y[j]);
     }
-    __syncthreads();
+    dft_twiddle<P, S, 1, 1>(y);
+#pragma unroll
+    for (int k = 0; k < P; k++) {
+        C z[S];
+#pragma unroll
+        for (int j = 0; j < S; j++) z[j] = y[j][k];
+        Dft<S, C>::go(z);
+#pragma unroll
+        for (int j = 0; j < S; j++) v[k + P * j] = z[j];
+    }
 }
+template <typename C> struct Dft<8, C> { __device__ static __forceinline__ void go(C* v) { dft_split<4, 2>(v); } };
+template <typename C> struct Dft<16, C> { __device__ static __forceinline__ void go(C* v) { dft_split<4, 4>(v); } };
+template <typename C> struct Dft<32, C> { __device__ static __forceinline__ void go(C* v) { dft_split<8, 4>(v); } };
 
-// Radix-8 pass (EPT a multiple of 8): eight points at stride N/8, twiddled, an
-// 8-point DFT as two 4-point DFTs of the even and odd points combined with the
-// eighth roots of unity, written back in natural order.
-template <int EPT, typename R, int TPB = FFT_THREADS>
-__device__ __forceinline__ void fft_pass_r8(cplx_t<R>* buf, int N, int Ns, int sign, const cplx_t<R>* __restrict__ tw) {
-    typedef cplx_t<R> C;
-    constexpr int NB = EPT / 8;
-    const int tid = threadIdx.x;
-    const int q8 = N >> 3;
-    const R h = (R)0.70710678118654752440;    // 1/sqrt(2)
-    C v[NB][8];
+// A pass of radix Q after passes of product NS: its twiddles (tw: the pass's
+// table), read before the exchange that precedes it, and the pass with them.
+template <int N, int Q, int NS, typename C>
+__device__ __forceinline__ void fft_tw(C* w, int t, const C* __restrict__ tw) {
+    constexpr int E = FftPlan<N>::E, T = N / E, B = E / Q;
 #pragma unroll
-    for (int q = 0; q < NB; q++) {
-        const int b = tid + TPB * q;
-        const int line = b / q8, j = b - line * q8;
-        const C* src = buf + line * N + j;
+    for (int q = 0; q < B; q++)
 #pragma unroll
-        for (int r = 0; r < 8; r++) v[q][r] = src[r * q8];
-    }
-    __syncthreads();
-    // s*i*z: the 4-point DFT's and W8's imaginary unit with the transform's sign
-    auto si = [sign](C z) __attribute__((always_inline)) {
-        return sign < 0 ? cmake<R>(z.y, -z.x) : cmake<R>(-z.y, z.x);
-    };
+        for (int r = 1; r < Q; r++) w[q * Q + r] = tw[(r - 1) * NS + (t + T * q) % NS];
+}
+template <int N, int Q, int NS, typename C>
+__device__ __forceinline__ void fft_pass(C (&v)[FftPlan<N>::E], int t, const C* __restrict__ tw) {
+    constexpr int E = FftPlan<N>::E, T = N / E, B = E / Q;
 #pragma unroll
-    for (int q = 0; q < NB; q++) {
-        const int b = tid + TPB * q;
-        const int line = b / q8, j = b - line * q8;
-        const int k = j % Ns;
-        if (Ns > 1) {
-            const int step = N / (Ns * 8);
+    for (int q = 0; q < B; q++) {
+        C z[Q];
+        const int k = (t + T * q) % NS;
 #pragma unroll
-            for (int r = 1; r < 8; r++) v[q][r] = cmul(v[q][r], tw_get(tw, k * r * step, sign));
+        for (int r = 0; r < Q; r++) {
+            z[r] = v[q + r * B];
+            if (NS > 1 && r > 0) z[r] = cmul(z[r], tw[q * Q + r]);
         }
-        // 4-point DFTs of the even (0, 2, 4, 6) and odd (1, 3, 5, 7) points
-        const C e0 = cadd(v[q][0], v[q][4]), e1 = csub(v[q][0], v[q][4]);
-        const C e2 = cadd(v[q][2], v[q][6]), e3 = si(csub(v[q][2], v[q][6]));
-        const C E0 = cadd(e0, e2), E1 = cadd(e1, e3), E2 = csub(e0, e2), E3 = csub(e1, e3);
-        const C o0 = cadd(v[q][1], v[q][5]), o1 = csub(v[q][1], v[q][5]);
-        const C o2 = cadd(v[q][3], v[q][7]), o3 = si(csub(v[q][3], v[q][7]));
-        C O0 = cadd(o0, o2), O1 = cadd(o1, o3), O2 = csub(o0, o2), O3 = csub(o1, o3);
-        // times W8^m = exp(s i pi m / 4), m = 1, 2, 3
-        O1 = crs(h, cadd(O1, si(O1)));
-        O2 = si(O2);
-        O3 = crs(h, csub(si(O3), O3));
-        C* dst = buf + line * N + (j / Ns) * Ns * 8 + k;
-        dst[0] = cadd(E0, O0);
-        dst[Ns] = cadd(E1, O1);
-        dst[2 * Ns] = cadd(E2, O2);
-        dst[3 * Ns] = cadd(E3, O3);
-        dst[4 * Ns] = csub(E0, O0);
-        dst[5 * Ns] = csub(E1, O1);
-        dst[6 * Ns] = csub(E2, O2);
-        dst[7 * Ns] = csub(E3, O3);
-    }
-    __syncthreads();
-}
-
-// In-place transform of the TOT/N lines held in buf (N a power of two).
-template <int EPT, typename R, int TPB = FFT_THREADS>
-__device__ __forceinline__ void fft_lds(cplx_t<R>* buf, int N, int log2N, int sign, const cplx_t<R>* __restrict__ tw) {
-    int Ns = 1;
-    if constexpr (EPT % 8 == 0) {
-        // radix-8 passes while three or more factors of two remain, then one
-        // radix-4 or radix-2 pass (the Stockham passes take the radices in any order)
-        int rem = log2N;
-        for (; rem >= 3; rem -= 3) {
-            fft_pass_r8<EPT, R, TPB>(buf, N, Ns, sign, tw);
-            Ns *= 8;
-        }
-        if (rem == 2) fft_pass_r4<EPT, R, TPB>(buf, N, Ns, sign, tw);
-        else if (rem == 1) fft_pass_r2<EPT, R, TPB>(buf, N, Ns, sign, tw);
-        return;
-    }
-    if (log2N & 1) {
-        fft_pass_r2<EPT, R, TPB>(buf, N, Ns, sign, tw);
-        Ns = 2;
-    }
-    while (Ns < N) {
-        fft_pass_r4<EPT, R, TPB>(buf, N, Ns, sign, tw);
-        Ns *= 4;
+        Dft<Q, C>::go(z);
+#pragma unroll
+        for (int r = 0; r < Q; r++) v[q + r * B] = z[r];
     }
 }
 
-// Twiddle table exp(-2 pi i k / N), k < N, cached per N on the device.
-const double2* fft_twiddles(int N);
-const float2* fft_twiddles_f(int N);
+template <int T>
+__device__ __forceinline__ void fft_sync() {
+    if constexpr (T > 64) __syncthreads();
+    else {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+
+// The results of a pass of radix Q (after passes of product NS) to natural
+// order: value j*Q-block ... of butterfly j goes to (j/NS)*NS*Q + j%NS + r*NS.
+// lds: the line's FftShape::LS bytes.
+template <int N, int Q, int NS, typename C>
+__device__ __forceinline__ void fft_exchange(C (&v)[FftPlan<N>::E], int t, void* lds) {
+    constexpr int E = FftPlan<N>::E, T = N / E, B = E / Q;
+    // value r of butterfly t + T*q goes to place st + (r*NS + q*T*Q), value e
+    // comes from t + T*e: the low four bits of the two terms do not carry, so
+    // the padding splits into that of the thread and a constant
+    static_assert(B == 1 || (T % NS == 0 && (T * Q) % 16 == 0), "places of a butterfly");
+    constexpr auto pad = [](int p) { return p + (p >> 4); };
+    const int st = pad((t / NS) * NS * Q + t % NS), ld = pad(t);
+    constexpr auto so = [pad](int e) { return pad((e / B) * NS + (e % B) * T * Q); };
+    constexpr auto lo = [pad](int e) { return pad(T * e); };
+    if constexpr (!fft_parts<N, C>()) {
+        C* const s = static_cast<C*>(lds);
+#pragma unroll
+        for (int e = 0; e < E; e++) s[st + so(e)] = v[e];
+        fft_sync<T>();
+#pragma unroll
+        for (int e = 0; e < E; e++) v[e] = s[ld + lo(e)];
+        fft_sync<T>();
+    } else {
+        auto* const s = static_cast<decltype(v[0].x)*>(lds);
+#pragma unroll
+        for (int e = 0; e < E; e++) s[st + so(e)] = v[e].x;
+        fft_sync<T>();
+#pragma unroll
+        for (int e = 0; e < E; e++) v[e].x = s[ld + lo(e)];
+        fft_sync<T>();
+#pragma unroll
+        for (int e = 0; e < E; e++) s[st + so(e)] = v[e].y;
+        fft_sync<T>();
+#pragma unroll
+        for (int e = 0; e < E; e++) v[e].y = s[ld + lo(e)];
+        fft_sync<T>();
+    }
+}
+
+// Transform of the line held by threads t = 0..T-1, v[e] = point t + T*e; sign < 0 forward, > 0 backward.
+template <int N, typename C>
+__device__ __forceinline__ void fft_line(C (&v)[FftPlan<N>::E], int t, void* lds, int sign, const C* __restrict__ tw) {
+    typedef FftPlan<N> P;
+    if (sign > 0) {
+#pragma unroll
+        for (int e = 0; e < P::E; e++) v[e].y = -v[e].y;
+    }
+    C w[P::E];
+    fft_pass<N, P::R0, 1>(v, t, w);
+    if constexpr (P::R1 > 1) {
+        fft_tw<N, P::R1, P::R0>(w, t, tw);
+        fft_exchange<N, P::R0, 1>(v, t, lds);
+        fft_pass<N, P::R1, P::R0>(v, t, w);
+    }
+    if constexpr (P::R2 > 1) {
+        fft_tw<N, P::R2, P::R0 * P::R1>(w, t, tw + (P::R1 - 1) * P::R0);
+        fft_exchange<N, P::R1, P::R0>(v, t, lds);
+        fft_pass<N, P::R2, P::R0 * P::R1>(v, t, w);
+    }
+    if (sign > 0) {
+#pragma unroll
+        for (int e = 0; e < P::E; e++) v[e].y = -v[e].y;
+    }
+}
 
 }  // namespace chimera
