@@ -154,6 +154,7 @@ constexpr size_t gb_lds_bytes(int WN, int GX) {
 // remainder) and the host has checked that every offset of the launch fits 31
 // bits (FbGemmArgs::buf_ok); the other stages take the guarded form.
 typedef float ch_vf2 __attribute__((ext_vector_type(2)));
+typedef unsigned int ch_vu4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t ch_rsrc(const void* p) {
     // raw buffer (stride 0), the whole 32-bit offset range, gfx9 word 3
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)0xFFFFFFFFu, 0x00020000);
@@ -508,11 +509,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t ch_rsrc_n(const void* p, uint3
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)n, 0x00020000);
 }
 
-__device__ __forceinline__ void stb_c(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, double2 v) {
-    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-    ch_vd2 w;
-    w.x = v.x, w.y = v.y;
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, w), r, (int)voff, (int)soff, 0);
+// 16-byte store.  Its offset stands whole in the vector register: a store whose
+// scalar offset is a register may still be reading its data when the next
+// instruction writes them, and the compiler puts the wait states between the
+// two only where the scalar offset is a constant.
+__device__ __forceinline__ void stb_16(__amdgpu_buffer_rsrc_t r, uint32_t voff, ch_vu4 v) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)voff, 0, 0);
 }
 
 // Epilogue of a tile wholly inside the output: the same values as
@@ -536,7 +538,7 @@ __device__ __forceinline__ void gemm_epilogue_full(const FbJob& J, const FbGemmA
         const __amdgpu_buffer_rsrc_t r1 = ch_rsrc(O.poiss_np1), r0 = ch_rsrc(O.poiss_n), rw = ch_rsrc(O.poiss_w2);
 #pragma unroll
         for (int j = 0; j < WN; j++) {
-            const uint32_t sj = (uint32_t)(16 * j * g.ldo * (int64_t)sizeof(double2));
+            const uint32_t sj = (uint32_t)(16 * j * g.ldo * (int64_t)sizeof(double2)), vj = v0 + sj;
 #pragma unroll
             for (int b = 0; b < NE; b += EB) {
                 double2 v[EB], dg[EB], pv[EB], n1[EB], nn[EB];
@@ -571,7 +573,7 @@ __device__ __forceinline__ void gemm_epilogue_full(const FbJob& J, const FbGemmA
 #pragma unroll
                 for (int e = 0; e < EB; e++) {
                     const int i = (b + e) / 2, h = (b + e) % 2;
-                    stb_c(rp, v0 + (uint32_t)(8 * i + 4 * h) * 16u, sj, v[e]);
+                    stb_16(rp, vj + (uint32_t)(8 * i + 4 * h) * 16u, __builtin_bit_cast(ch_vu4, v[e]));
                 }
             }
         }
