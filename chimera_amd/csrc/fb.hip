@@ -17,6 +17,7 @@
 #include <cmath>
 #include <cstdio>
 #include <string>
+#include <tuple>
 #include <complex>
 #include <map>
 #include <mutex>
@@ -75,6 +76,7 @@ template int32_t make_phase<float>(float2*, const double*, double, double, int, 
 // that a lane's items (0,1) and (2,3) are the (re, im) of x = c and x = c + 4
 // with c = l/16.
 constexpr int GB_X = 64, GB_K = 16, GB_THREADS = 256;
+constexpr int GBB_K = 32, GBB_RS = GBB_K + 8;          // split BF16: K per stage; LDS row stride in BF16
 // LDS row padding in doubles: rows 16 doubles (128 B) apart modulo 256 B put the
 // two rows that a half-wave reads in one ds_read_b64 on disjoint bank halves.
 constexpr int GB_PAD = 16;
@@ -732,13 +734,14 @@ __global__ void __launch_bounds__(GB_THREADS, gemm_pipe_occ(NACC, WN)) k_fb_gemm
 // The kind of the segments of a job list: 0: T(a0); 1: i T(a0) + s T(a1), s =
 // +-1; plus 2 where some K is no multiple of GB_K; -1: of neither kind, or too
 // large for 31-bit offsets (k_fb_gemm).
-static int gemm_pipe_kind(const std::vector<FbJob>& jobs, int buf_ok) {
+template <typename R>
+static int gemm_pipe_kind(const std::vector<FbJobT<R>>& jobs, int buf_ok) {
     int kind = -2, rem = 0;
     for (const auto& j : jobs) {
         if (j.K < 1) return -1;
-        rem |= j.K % GB_K != 0;
+        rem |= j.K % (sizeof(R) == 8 ? GB_K : GBB_K) != 0;
         for (int q = 0; q < j.nseg; q++) {
-            const FbSeg& s = j.seg[q];
+            const FbSegT<R>& s = j.seg[q];
             const int k = !s.a1 && s.c0.x == 1.0 && s.c0.y == 0.0 ? 0
                         : s.a1 && s.c0.x == 0.0 && s.c0.y == 1.0 && fabs(s.c1.x) == 1.0 && s.c1.y == 0.0 ? 1 : -1;
             if (k < 0 || (kind != -2 && k != kind) || s.ldd != j.seg[0].ldd) return -1;
@@ -868,6 +871,8 @@ template <int NACC, int WN, int GX = GB_X>
 static int32_t launch_gemm_variant_f32(const FbJobT<float>* dj, size_t njobs, int maxN, const FbGemmArgs& g);
 template <int NACC, int WN, int GX = GB_X>
 static int32_t launch_gemm_variant_bf16(const FbJobT<float>* dj, size_t njobs, int maxN, const FbGemmArgs& g);
+template <int NACC, int WN>
+static int32_t launch_gemm_bf16_pipe(const FbJobT<float>* dj, size_t njobs, int maxN, const FbGemmArgs& g);
 
 // Form of the mixed-precision GEMMs: split-BF16 (six products, the default)
 // or FP32 MFMA; process-wide, set by chimera_set_mixed_gemm.
@@ -898,6 +903,14 @@ static int32_t gemm_tile_launch(const FbJob* dj, size_t nj, int maxN, const FbGe
 static int32_t gemm_tile_launch(const FbJobT<float>* dj, size_t nj, int maxN, const FbGemmArgs& g, int nacc,
                                 int tile) {
     if (g_mixed_gemm.load() == MIXED_GEMM_BF16X6) {
+        if (g.pipe >= 0 && tile < GT_H) {
+            if (nacc == 2)
+                return tile == GT_W4 ? ST_EUNSUP : tile == GT_W2 ? launch_gemm_bf16_pipe<2, 2>(dj, nj, maxN, g)
+                                                                 : launch_gemm_bf16_pipe<2, 1>(dj, nj, maxN, g);
+            return tile == GT_W4   ? launch_gemm_bf16_pipe<1, 4>(dj, nj, maxN, g)
+                   : tile == GT_W2 ? launch_gemm_bf16_pipe<1, 2>(dj, nj, maxN, g)
+                                   : launch_gemm_bf16_pipe<1, 1>(dj, nj, maxN, g);
+        }
         if (nacc == 1) {
             switch (tile) {
                 case GT_W4: return launch_gemm_variant_bf16<1, 4>(dj, nj, maxN, g);
@@ -1059,7 +1072,7 @@ int32_t launch_fb_gemm<double>(const std::vector<FbJob>& jobs, const FbGemmArgs&
         for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
         const FbJob* dj = static_cast<const FbJob*>(device_table(js.data(), js.size() * sizeof(FbJob)));
         if (!dj) return ST_ENOMEM;
-        g.pipe = gemm_pipe_kind(js, g.buf_ok);
+        g.pipe = gemm_pipe_kind<double>(js, g.buf_ok);
         int tile = gemm_choose_tile<FbJob>(dj, js, maxN, g, pass + 1, 8);
         if (g.pipe < 0 && tile < GT_H) tile = GT_H;
         CH_TRY(gemm_tile_launch(dj, js.size(), maxN, g, pass + 1, tile));
@@ -1274,7 +1287,6 @@ static int32_t launch_gemm_variant_f32(const FbJobT<float>* dj, size_t njobs, in
 // 16-byte read then hit disjoint banks).  One LDS buffer: the next stage is
 // loaded into registers while the MFMAs of this one run.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-constexpr int GBB_K = 32, GBB_RS = GBB_K + 8;          // K per stage; LDS row stride in BF16
 
 // v = h + m + l exactly (finite v of normal magnitude); pieces as BF16 bit
 // patterns.  Each piece is the round-to-nearest-even BF16 of what is left
@@ -1486,6 +1498,355 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm_bf16(const FbJobT<flo
     gemm_epilogue<float, NACC, WN, NI>(J, g, acc0, acc1, Ncol, n0, x0, lane, wr, wc);
 }
 
+// ---- split BF16, tiles of 64 complex x of large launches
+//
+// The same tile, pieces, products and order as k_fb_gemm_bf16, for the two
+// kinds of segments of k_fb_gemm_pipe.  There the vector units split every
+// element of D again in each of the nx / 64 blocks that read it, and the
+// split stood between two barriers, beside no MFMA of its own block.  Here
+// k_split_d lays the pieces of D out once per call as the stages read them
+// (stage, piece, column, 32 k; zeros past K and Ncol), the pieces of A are
+// formed while the MFMAs of the previous stage run, and only the LDS stores
+// stand between the barriers; with the XCD mapping, the full-tile epilogue and
+// the loop without address arithmetic of k_fb_gemm_pipe.  Forward Hankel
+// transforms at 8192 x 512, four modes: 964 -> 690 us, 153 TFLOP/s of FP32
+// products where a plain BF16 product reaches 1110 / 6 = 185; Poisson
+// correction at 4096 x 256, three modes: 267 -> 174 us.
+template <int WN>
+struct GemmPipeBf {
+    static constexpr int BN = 32 * WN, ROWS = 2 * GB_X;
+    static constexpr int PA = ROWS * GBB_RS, PD = BN * GBB_RS;
+    static constexpr int KA = GBB_K * GB_X / GB_THREADS;
+    static constexpr int ND = WN == 1 ? 1 : WN / 2;         // 16-byte chunks of a piece of D per thread
+};
+struct SplitMat {
+    const float* D;
+    uint16_t* out;
+    int64_t ldd;
+    int K, Ncol, npad;
+};
+constexpr int gbb_npad(int Ncol) { return (Ncol + 127) / 128 * 128; }
+constexpr int64_t gbb_bytes(int K, int Ncol) { return (int64_t)((K + GBB_K - 1) / GBB_K) * 3 * gbb_npad(Ncol) * 64; }
+
+// Pieces of the matrices of a launch: thread = 8 k of one column.
+__global__ void __launch_bounds__(256) k_split_d(const SplitMat* __restrict__ mats) {
+    const SplitMat m = mats[blockIdx.y];
+    const int stages = (m.K + GBB_K - 1) / GBB_K;
+    const int64_t n = (int64_t)stages * m.npad * 4;
+    for (int64_t e = blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+        const int part = (int)(e & 3), col = (int)((e >> 2) % m.npad), st = (int)((e >> 2) / m.npad);
+        const int k = st * GBB_K + part * 8;
+        uint16_t h[8], md[8], l[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const float v = col < m.Ncol && k + q < m.K ? m.D[k + q + m.ldd * col] : 0.f;
+            split3_bf16(v, h[q], md[q], l[q]);
+        }
+        uint16_t* const o = m.out + ((int64_t)st * 3 * m.npad + col) * GBB_K + part * 8;
+        const int64_t pp = (int64_t)m.npad * GBB_K;
+        lds_store_bf16<8>(o, h);
+        lds_store_bf16<8>(o + pp, md);
+        lds_store_bf16<8>(o + 2 * pp, l);
+    }
+}
+
+__device__ __forceinline__ ch_vu4 ldb_u4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(ch_vu4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
+}
+struct CPair { float2 a, b; };          // x and x + 1
+__device__ __forceinline__ CPair ldb_cc(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(CPair, ldb_u4(r, voff, soff));
+}
+
+// gemm_epilogue_full for complex64: a lane's outputs are pairs of neighbours in x.
+template <int NACC, int WN, int EB>
+__device__ __forceinline__ void gemm_epilogue_full_f(const FbJobT<float>& J, const FbGemmArgs& g,
+                                                     const flt4 (&acc0)[4][WN], const flt4 (&acc1)[4][NACC == 2 ? WN : 1],
+                                                     int n0, int x0, int lane, int wr, int wc) {
+    const int xl = x0 + wr * 32 + 2 * (lane >> 4);
+    const uint32_t v0 = (uint32_t)((xl + g.ldo * (n0 + wc * 16 * WN + (lane & 15))) * (int64_t)sizeof(float2));
+    const bool beta = J.beta != 0;
+    const float dti = (float)g.dt_inv;
+    for (int o = 0; o < J.nout; o++) {
+        const FbOutT<float> O = J.out[o];
+        const float2 al0 = to_f(O.alpha0), al1 = to_f(O.alpha1), gam = to_f(O.gamma);
+        const __amdgpu_buffer_rsrc_t rp = ch_rsrc(O.p), rd = ch_rsrc(O.diag), rs = ch_rsrc(O.scale);
+        const __amdgpu_buffer_rsrc_t r1 = ch_rsrc(O.poiss_np1), r0 = ch_rsrc(O.poiss_n), rw = ch_rsrc(O.poiss_w2);
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+            const uint32_t sj = (uint32_t)(16 * j * g.ldo * (int64_t)sizeof(float2)), vj = v0 + sj;
+#pragma unroll
+            for (int b = 0; b < 4; b += EB) {
+                CPair dg[EB], pv[EB], n1[EB], nn[EB];
+                float2 sc[EB], w2[EB];
+                double kxa[EB], kxb[EB];
+#pragma unroll
+                for (int e = 0; e < EB; e++) {
+                    const uint32_t ve = v0 + (uint32_t)(8 * (b + e)) * 8u;
+                    if (O.diag) {
+                        dg[e] = ldb_cc(rd, ve, sj);
+                        kxa[e] = g.kx[xl + 8 * (b + e)];
+                        kxb[e] = g.kx[xl + 8 * (b + e) + 1];
+                    }
+                    if (O.scale) sc[e] = ldb_c(rs, ve / 2, sj / 2, float2{});
+                    if (O.poiss) {
+                        n1[e] = ldb_cc(r1, ve, sj);
+                        nn[e] = ldb_cc(r0, ve, sj);
+                        w2[e] = ldb_c(rw, ve / 2, sj / 2, float2{});
+                    }
+                    if (O.poiss || beta) pv[e] = ldb_cc(rp, ve, sj);
+                }
+#pragma unroll
+                for (int e = 0; e < EB; e++) {
+                    const int i = b + e;
+                    auto one = [&](int h, float2 dgv, double kx, float scv, float2 pvv, float2 n1v, float2 nnv,
+                                   float w2v) __attribute__((always_inline)) {
+                        float2 w = cmul(al0, cmake<float>(acc0[i][j][2 * h], acc0[i][j][2 * h + 1]));
+                        if constexpr (NACC == 2)
+                            w = cadd(w, cmul(al1, cmake<float>(acc1[i][j][2 * h], acc1[i][j][2 * h + 1])));
+                        if (O.diag) w = cadd(w, crs((float)kx, cmul(gam, dgv)));
+                        if (O.scale) w = crs(scv, w);
+                        // maxwell_solvers.f90:153-158: J += (v + (g_np1 - g_n)*dt_inv)*w2_inv
+                        if (O.poiss) w = cadd(pvv, crs(w2v, cadd(w, crs(dti, csub(n1v, nnv)))));
+                        else if (beta) w = cadd(pvv, w);
+                        return w;
+                    };
+                    CPair w;
+                    w.a = one(0, dg[e].a, kxa[e], sc[e].x, pv[e].a, n1[e].a, nn[e].a, w2[e].x);
+                    w.b = one(1, dg[e].b, kxb[e], sc[e].y, pv[e].b, n1[e].b, nn[e].b, w2[e].y);
+                    stb_16(rp, vj + (uint32_t)(8 * i) * 8u, __builtin_bit_cast(ch_vu4, w));
+                }
+            }
+        }
+    }
+}
+
+// KR: some K of the launch is no multiple of GBB_K.
+template <int NACC, int WN, bool A1, bool KR>
+__global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm_bf16_pipe(const FbJobT<float>* __restrict__ jobs,
+                                                                     FbGemmArgs g, int nx8, int nyt) {
+    typedef GemmPipeBf<WN> G;
+    typedef FbSegT<float> Seg;
+    constexpr int NI = 4, BN = G::BN, KA = G::KA, ND = G::ND;
+    // blocks to tiles as in k_fb_gemm_pipe
+    int id = blockIdx.x >> 3;
+    const int yt = id % nyt;
+    id /= nyt;
+    const int n0 = yt * BN, x0 = ((id % nx8) * 8 + (blockIdx.x & 7)) * GB_X;
+    const FbJobT<float>& J = jobs[id / nx8];
+    const int Ncol = J.Ncol, K = J.K, nseg = J.nseg;
+    if (n0 >= Ncol || x0 >= g.nx) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave & 1, wc = wave >> 1;
+
+    extern __shared__ __align__(16) unsigned char gbq_smem[];
+    uint16_t* const As = reinterpret_cast<uint16_t*>(gbq_smem);     // [3][ROWS][GBB_RS]
+    uint16_t* const Ds = As + 3 * G::PA;                             // [3][BN][GBB_RS]
+
+    flt4 acc0[NI][WN], acc1[NI][NACC == 2 ? WN : 1];
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int j = 0; j < WN; j++) acc0[i][j] = flt4{0.f, 0.f, 0.f, 0.f};
+
+    const int sps = (K + GBB_K - 1) / GBB_K, nst = sps * nseg;
+    const Seg S0 = J.seg[0], S1 = J.seg[nseg > 1 ? 1 : 0];
+    const uint32_t row = (uint32_t)(g.lda * sizeof(float2));
+    const uint32_t la0 = seg_lane_a(S0, min(x0 + lane, g.nx - 1), g.nx, g.lda, 0);
+    const uint32_t la1 = seg_lane_a(S1, min(x0 + lane, g.nx - 1), g.nx, g.lda, 0);
+    const int kb = KA * wave;
+    const uint32_t dpiece = (uint32_t)gbb_npad(Ncol) * 64u;
+    const uint32_t lcol = (uint32_t)n0 * 64u + (uint32_t)(WN == 1 ? tid & 127 : tid) * 16u;
+    float2 ra[KA], rb[A1 ? KA : 1];
+    ch_vu4 pa[6], rd[3][ND];
+    // A of stage t: k = k0 + kb + q of x = x0 + lane
+    auto fetch_a = [&](int t) __attribute__((always_inline)) {
+        const bool s = t >= sps;
+        const int k0 = (s ? t - sps : t) * GBB_K;
+        const __amdgpu_buffer_rsrc_t rs_a = ch_rsrc(s ? S1.a0 : S0.a0);
+        const uint32_t la = s ? la1 : la0;
+#pragma unroll
+        for (int q = 0; q < KA; q++)
+            ra[q] = ldb_c(rs_a, la, (uint32_t)(KR ? min(k0 + kb + q, K - 1) : k0 + kb + q) * row, float2{});
+        if constexpr (A1) {
+            const __amdgpu_buffer_rsrc_t rs_b = ch_rsrc(s ? S1.a1 : S0.a1);
+#pragma unroll
+            for (int q = 0; q < KA; q++)
+                rb[q] = ldb_c(rs_b, la, (uint32_t)(KR ? min(k0 + kb + q, K - 1) : k0 + kb + q) * row, float2{});
+        }
+    };
+    auto fetch_d = [&](int t) __attribute__((always_inline)) {
+        const bool s = t >= sps;
+        const __amdgpu_buffer_rsrc_t rs_d = ch_rsrc(s ? S1.ds : S0.ds);
+        const uint32_t so = (uint32_t)(s ? t - sps : t) * 3u * dpiece;
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+#pragma unroll
+            for (int i = 0; i < ND; i++) rd[p][i] = ldb_u4(rs_d, lcol, so + p * dpiece + (uint32_t)i * 4096u);
+    };
+    // the pieces of A of stage t: rows 2*lane (re: pa[0..2]) and 2*lane + 1 (im)
+    auto split_a = [&](int t) __attribute__((always_inline)) {
+        const bool s = t >= sps;
+        const int k0 = (s ? t - sps : t) * GBB_K;
+        const bool refl = s ? S1.refl : S0.refl;            // T(v) = (-v.x, v.y)
+        const float sr = refl ? -1.f : 1.f;
+        const float sg = A1 ? (float)(s ? S1.c1.x : S0.c1.x) : 0.f, sgx = sg * sr;
+        uint16_t pc[6][KA];
+#pragma unroll
+        for (int q = 0; q < KA; q++) {
+            float2 v;
+            if constexpr (A1) v = cmkf(fmaf(sgx, rb[q].x, -ra[q].y), fmaf(sg, rb[q].y, sr * ra[q].x));
+            else v = cmkf(sr * ra[q].x, ra[q].y);
+            if (KR && k0 + kb + q >= K) v = cmkf(0.f, 0.f);
+            split3_bf16(v.x, pc[0][q], pc[1][q], pc[2][q]);
+            split3_bf16(v.y, pc[3][q], pc[4][q], pc[5][q]);
+        }
+#pragma unroll
+        for (int p = 0; p < 6; p++)
+#pragma unroll
+            for (int w = 0; w < 4; w++) pa[p][w] = (uint32_t)pc[p][2 * w] | ((uint32_t)pc[p][2 * w + 1] << 16);
+    };
+    auto store = [&]() __attribute__((always_inline)) {
+        uint16_t* const a = As + 2 * lane * GBB_RS + kb;
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            *reinterpret_cast<ch_vu4*>(a + p * G::PA) = pa[p];
+            *reinterpret_cast<ch_vu4*>(a + GBB_RS + p * G::PA) = pa[3 + p];
+        }
+        if (WN > 1 || tid < 128) {
+            uint16_t* const d = Ds + (tid >> 2) * GBB_RS + (tid & 3) * 8;
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+#pragma unroll
+                for (int i = 0; i < ND; i++) *reinterpret_cast<ch_vu4*>(d + p * G::PD + i * 64 * GBB_RS) = rd[p][i];
+        }
+    };
+    const uint16_t* const ard = As + (wr * 64 + (lane & 15)) * GBB_RS + 8 * (lane >> 4);
+    const uint16_t* const drd = Ds + (wc * 16 * WN + (lane & 15)) * GBB_RS + 8 * (lane >> 4);
+    auto run = [&](flt4 (&acc)[NI][WN], int tb, int te) __attribute__((always_inline)) {
+        for (int t = tb; t < te; t++) {
+            bf16x8 ah[NI], am[NI], al[NI];
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const uint16_t* a = ard + 16 * i * GBB_RS;
+                ah[i] = *reinterpret_cast<const bf16x8*>(a);
+                am[i] = *reinterpret_cast<const bf16x8*>(a + G::PA);
+                al[i] = *reinterpret_cast<const bf16x8*>(a + 2 * G::PA);
+            }
+            split_a(min(t + 1, nst - 1));
+            fetch_a(min(t + 2, nst - 1));
+#pragma unroll
+            for (int j = 0; j < WN; j++) {
+                const uint16_t* d = drd + 16 * j * GBB_RS;
+                const bf16x8 bh = *reinterpret_cast<const bf16x8*>(d);
+                const bf16x8 bm = *reinterpret_cast<const bf16x8*>(d + G::PD);
+                const bf16x8 bl = *reinterpret_cast<const bf16x8*>(d + 2 * G::PD);
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    flt4 c = acc[i][j];
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh, c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am[i], bm, c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl, c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am[i], bh, c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bm, c, 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh, c, 0, 0, 0);
+                }
+            }
+            __syncthreads();
+            store();
+            fetch_d(min(t + 2, nst - 1));
+            __syncthreads();
+        }
+    };
+    if (nst > 0) {
+        fetch_a(0);
+        fetch_d(0);
+        split_a(0);
+        store();
+        fetch_a(min(1, nst - 1));
+        fetch_d(min(1, nst - 1));
+        __syncthreads();
+        run(acc0, 0, NACC == 2 ? sps : nst);
+    }
+    if constexpr (NACC == 2) {
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+            for (int j = 0; j < WN; j++) acc1[i][j] = flt4{0.f, 0.f, 0.f, 0.f};
+        run(acc1, sps, nst);
+    }
+    if (x0 + GB_X <= g.nx && n0 + BN <= Ncol) {
+        gemm_epilogue_full_f<NACC, WN, (NACC * WN >= 4 ? 2 : 4)>(J, g, acc0, acc1, n0, x0, lane, wr, wc);
+    } else {
+        gemm_epilogue_serial<float, NACC, WN, NI>(J, g, acc0, acc1, Ncol, n0, x0, lane, wr, wc);
+    }
+}
+
+template <int NACC, int WN, bool A1, bool KR>
+static int32_t launch_gemm_bf16_pipe_k(const FbJobT<float>* dj, size_t njobs, int maxN, const FbGemmArgs& g) {
+    constexpr size_t lds = gb_lds_bytes_bf16(WN, GB_X);
+    static bool attr = false;
+    if (!attr) {
+        CH_HIP(hipFuncSetAttribute((const void*)k_fb_gemm_bf16_pipe<NACC, WN, A1, KR>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        attr = true;
+    }
+    const int nx8 = (g.nx + 8 * GB_X - 1) / (8 * GB_X), nyt = (maxN + 32 * WN - 1) / (32 * WN);
+    const unsigned grid = (unsigned)((size_t)nx8 * 8 * nyt * njobs);
+    hipLaunchKernelGGL((k_fb_gemm_bf16_pipe<NACC, WN, A1, KR>), grid, GB_THREADS, lds, stream(), dj, g, nx8, nyt);
+    CH_LAUNCH_CHECK("k_fb_gemm_bf16_pipe");
+    return ST_OK;
+}
+
+template <int NACC, int WN>
+static int32_t launch_gemm_bf16_pipe(const FbJobT<float>* dj, size_t njobs, int maxN, const FbGemmArgs& g) {
+    switch (g.pipe) {
+        case 0: return launch_gemm_bf16_pipe_k<NACC, WN, false, false>(dj, njobs, maxN, g);
+        case 1: return launch_gemm_bf16_pipe_k<NACC, WN, true, false>(dj, njobs, maxN, g);
+        case 2: return launch_gemm_bf16_pipe_k<NACC, WN, false, true>(dj, njobs, maxN, g);
+        default: return launch_gemm_bf16_pipe_k<NACC, WN, true, true>(dj, njobs, maxN, g);
+    }
+}
+
+// The pieces of every matrix of the jobs into scratch slot 17, and Seg::ds set;
+// false where the scratch has no room for them.
+static bool split_matrices(std::vector<FbJobT<float>>& js) {
+    typedef std::tuple<const float*, int64_t, int, int> Key;
+    std::map<Key, int64_t> at;
+    int64_t bytes = 0, most = 0;
+    for (const auto& j : js)
+        for (int q = 0; q < j.nseg; q++) {
+            const Key k(j.seg[q].D, j.seg[q].ldd, j.K, j.Ncol);
+            if (!at.emplace(k, bytes).second) continue;
+            const int64_t b = gbb_bytes(j.K, j.Ncol);
+            most = b > most ? b : most;
+            bytes += b;
+        }
+    if (most >= (int64_t)1 << 31) return false;
+    char* const p = static_cast<char*>(scratch(17, (size_t)bytes));
+    if (!p) return false;
+    std::vector<SplitMat> mats;
+    for (const auto& kv : at) {
+        SplitMat m;
+        memset(&m, 0, sizeof m);
+        m.D = std::get<0>(kv.first);
+        m.out = reinterpret_cast<uint16_t*>(p + kv.second);
+        m.ldd = std::get<1>(kv.first);
+        m.K = std::get<2>(kv.first);
+        m.Ncol = std::get<3>(kv.first);
+        m.npad = gbb_npad(m.Ncol);
+        mats.push_back(m);
+    }
+    for (auto& j : js)
+        for (int q = 0; q < j.nseg; q++)
+            j.seg[q].ds = p + at[Key(j.seg[q].D, j.seg[q].ldd, j.K, j.Ncol)];
+    const SplitMat* dm = static_cast<const SplitMat*>(device_table(mats.data(), mats.size() * sizeof(SplitMat)));
+    if (!dm) return false;
+    const dim3 grid((unsigned)((most / 192 * 4 + 255) / 256), (unsigned)mats.size());
+    hipLaunchKernelGGL(k_split_d, grid, 256, 0, stream(), dm);
+    return hipGetLastError() == hipSuccess;
+}
+
 template <int NACC, int WN, int GX>
 static int32_t launch_gemm_variant_bf16(const FbJobT<float>* dj, size_t njobs, int maxN, const FbGemmArgs& g) {
     constexpr int BN = 32 * WN;
@@ -1502,6 +1863,14 @@ static int32_t launch_gemm_variant_bf16(const FbJobT<float>* dj, size_t njobs, i
     return ST_OK;
 }
 
+// The split of the matrices is a launch more: for launches of at least 2^29
+// products of a real by a complex value (forward transform, matrices split in
+// the kernel and once per call, microseconds of the whole call, FFT included:
+// 1024 x 128 x 2 modes 29 and 31, 2048 x 128 x 2 39 and 40, 1024 x 256 x 3, 6e8
+// products, 66 and 54, 1024 x 500 x 2 114 and 77; Poisson correction 2048 x 128 x 2
+// 49 and 55, 4096 x 128 x 3 101 and 70).
+constexpr int64_t GEMM_SPLIT_WORK = (int64_t)1 << 29;
+
 template <>
 int32_t launch_fb_gemm<float>(const std::vector<FbJobT<float>>& jobs, const FbGemmArgs& g_in, int family) {
     if (jobs.empty()) return ST_OK;
@@ -1515,10 +1884,19 @@ int32_t launch_fb_gemm<float>(const std::vector<FbJobT<float>>& jobs, const FbGe
         one.clear();
     }
     for (int pass = 0; pass < 2; pass++) {
-        const std::vector<FbJobT<float>>& js = pass == 0 ? one : two;
+        std::vector<FbJobT<float>>& js = pass == 0 ? one : two;
         if (js.empty()) continue;
+        // the jobs of two segments first, so that the last blocks to start are short
+        std::stable_sort(js.begin(), js.end(),
+                         [](const FbJobT<float>& a, const FbJobT<float>& b) { return a.nseg > b.nseg; });
         int maxN = 0;
         for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
+        g.pipe = g_mixed_gemm.load() == MIXED_GEMM_BF16X6 ? gemm_pipe_kind<float>(js, g.buf_ok) : -1;
+        if (g.pipe >= 0) {
+            int64_t work = 0;
+            for (const auto& j : js) work += (int64_t)j.nseg * j.K * j.Ncol * g.nx;
+            if (work < GEMM_SPLIT_WORK || !split_matrices(js)) g.pipe = -1;
+        }
         const FbJobT<float>* dj =
             static_cast<const FbJobT<float>*>(device_table(js.data(), js.size() * sizeof(FbJobT<float>)));
         if (!dj) return ST_ENOMEM;
@@ -1540,6 +1918,7 @@ static FbSegT<R> seg(const cplx_t<R>* a0, double2 c0, const cplx_t<R>* a1, doubl
     s.c0 = c0;
     s.c1 = c1;
     s.D = D;
+    s.ds = nullptr;
     s.ldd = ldd;
     s.refl = refl;
     s.acc = acc;

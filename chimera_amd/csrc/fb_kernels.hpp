@@ -57,6 +57,7 @@ struct FbSegT {
     const C* a1;
     double2 c0, c1;
     const R* D;
+    const void* ds;                // set by launch_fb_gemm<float>: D in BF16 pieces (k_split_d)
     int64_t ldd;
     int refl;
     int acc;

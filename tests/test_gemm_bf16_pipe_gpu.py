@@ -1,0 +1,46 @@
+"""The split-BF16 GEMMs of large launches (matrices split once per call) at the
+edges of their tiles: x and column remainders in 128-, 64- and 32-column tiles,
+K no multiple of the 32-deep stage, both kinds of segments and one and two
+accumulators (rot, grad, div, graddiv), against the FP64 oracle; and the same
+bits from call to call.
+
+Bar 2e-6, that of the other tile tests: 6e-8 sqrt(2 K) for FP32 sums of two
+segments of K <= 544 products, with operands exact in FP32.
+"""
+import numpy as np
+import pytest
+
+from tests._cases import C, F, rel_l2, rng
+from tests.test_gemm_tiles_gpu import OPS, TOL32, _c8, say
+
+pytestmark = pytest.mark.gpu
+
+
+# 8190 x 160: 128-column tiles with 32 columns left, two x of the last tile
+# missing; 4100 x 300: K remainder 12; 1030 x 544: 64-column tiles; 520 x 520:
+# 32-column tiles, K remainder 8
+@pytest.mark.timeout(900)
+@pytest.mark.parametrize("nkx,nkr,nko,name", [(8190, 160, 1, "div"), (8190, 160, 1, "rot"), (4100, 300, 1, "grad"),
+                                              (4100, 300, 1, "graddiv"), (1030, 544, 1, "div"),
+                                              (1030, 544, 1, "grad"), (520, 520, 2, "graddiv"),
+                                              (520, 520, 2, "rot")])
+def test_edges(gpu, port, nkx, nkr, nko, name):
+    say(f"case: fb_{name} nkx={nkx} nkr={nkr} nko={nko}")
+    r = rng(9000 + nkx + nkr)
+    f4 = lambda a: np.asfortranarray(a.astype(np.float32 if a.dtype == float else np.complex64).astype(a.dtype))  # noqa: E731
+    kx = 2 * np.pi * np.fft.fftfreq(nkx, 1.0)
+    Dp, Dm = f4(F(r, nkr, nkr, nko + 2)), f4(F(r, nkr, nkr, nko + 2))
+    v, s = f4(C(r, nkx, nkr, nko + 1, 3)), f4(C(r, nkx, nkr, nko + 1))
+    if name == "graddiv":
+        out, inp = v, v
+        ref = port.fb_graddiv(v.copy(order="F"), Dp, Dm, kx)
+    else:
+        out = np.zeros((nkx, nkr, nko + 1) + (() if name == "div" else (3,)), complex, order="F")
+        inp = s if name == "grad" else v
+        ref = getattr(port, "fb_" + name)(out.copy(order="F"), inp, Dp, Dm, kx)
+    first = _c8(OPS[name], out.copy(order="F"), inp, Dp, Dm, kx, nko)
+    e = rel_l2(first, ref)
+    say(f"  mixed {e:.2e}")
+    assert e < TOL32
+    for _ in range(3):
+        assert np.array_equal(_c8(OPS[name], out.copy(order="F"), inp, Dp, Dm, kx, nko), first)
