@@ -4,7 +4,7 @@
 // fb_math.f90.
 //
 // Every dense contraction (Hankel matrices In/Out, the mode-coupling matrices
-// DpS2S/DmS2S) goes through ONE job-driven kernel, k_fb_gemm: a job is an
+// DpS2S/DmS2S) goes through job-driven kernels, k_fb_gemm*: a job is an
 // output mode of one operator, made of up to two K-segments
 //   P_s(x,k) = sum_k' A_s(x,k') D_s(k',k),   A_s = c0*T(a0) + c1*T(a1)
 // (T = identity, or the reflected conjugate -conj(v(-kx)) that stands for mode
