@@ -1051,6 +1051,27 @@ static int gemm_choose_tile(const J* dj, const std::vector<J>& js, int maxN, con
     return best;
 }
 
+// The launches of a job list: one, or one per kind where the list mixes the two
+// kinds and is large enough for the 64-complex-x tiles, whose pipeline takes one
+// kind (the curl's list of one accumulator: at 8192 x 512, four modes, 2.33 ms in
+// one launch of 32-complex-x tiles).
+template <typename R>
+static std::vector<std::vector<FbJobT<R>>> gemm_groups(const std::vector<FbJobT<R>>& js, const FbGemmArgs& g, int nacc) {
+    int maxN = 0;
+    for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
+    if (!g.buf_ok || js.empty() || gemm_pipe_kind<R>(js, 1) >= 0 ||
+        gemm_tile(g.nx, maxN, js.size(), sizeof(R) == 4 || nacc == 1) >= GT_H)
+        return {js};
+    std::vector<std::vector<FbJobT<R>>> gr(3), out;
+    for (const auto& j : js) {
+        const int k = gemm_pipe_kind<R>({j}, 1);
+        gr[k < 0 ? 2 : k & 1].push_back(j);
+    }
+    for (auto& v : gr)
+        if (!v.empty()) out.push_back(std::move(v));
+    return out;
+}
+
 template <>
 int32_t launch_fb_gemm<double>(const std::vector<FbJob>& jobs, const FbGemmArgs& g_in, int family) {
     if (jobs.empty()) return ST_OK;
@@ -1064,18 +1085,19 @@ int32_t launch_fb_gemm<double>(const std::vector<FbJob>& jobs, const FbGemmArgs&
         one.clear();
     }
     for (int pass = 0; pass < 2; pass++) {
-        std::vector<FbJob>& js = pass == 0 ? one : two;
-        if (js.empty()) continue;
-        // the jobs of two segments first, so that the last blocks to start are short
-        std::stable_sort(js.begin(), js.end(), [](const FbJob& a, const FbJob& b) { return a.nseg > b.nseg; });
-        int maxN = 0;
-        for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
-        const FbJob* dj = static_cast<const FbJob*>(device_table(js.data(), js.size() * sizeof(FbJob)));
-        if (!dj) return ST_ENOMEM;
-        g.pipe = gemm_pipe_kind<double>(js, g.buf_ok);
-        int tile = gemm_choose_tile<FbJob>(dj, js, maxN, g, pass + 1, 8);
-        if (g.pipe < 0 && tile < GT_H) tile = GT_H;
-        CH_TRY(gemm_tile_launch(dj, js.size(), maxN, g, pass + 1, tile));
+        for (std::vector<FbJob>& js : gemm_groups<double>(pass == 0 ? one : two, g, pass + 1)) {
+            if (js.empty()) continue;
+            // the jobs of two segments first, so that the last blocks to start are short
+            std::stable_sort(js.begin(), js.end(), [](const FbJob& a, const FbJob& b) { return a.nseg > b.nseg; });
+            int maxN = 0;
+            for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
+            const FbJob* dj = static_cast<const FbJob*>(device_table(js.data(), js.size() * sizeof(FbJob)));
+            if (!dj) return ST_ENOMEM;
+            g.pipe = gemm_pipe_kind<double>(js, g.buf_ok);
+            int tile = gemm_choose_tile<FbJob>(dj, js, maxN, g, pass + 1, 8);
+            if (g.pipe < 0 && tile < GT_H) tile = GT_H;
+            CH_TRY(gemm_tile_launch(dj, js.size(), maxN, g, pass + 1, tile));
+        }
     }
     return ST_OK;
 }
@@ -1884,25 +1906,26 @@ int32_t launch_fb_gemm<float>(const std::vector<FbJobT<float>>& jobs, const FbGe
         one.clear();
     }
     for (int pass = 0; pass < 2; pass++) {
-        std::vector<FbJobT<float>>& js = pass == 0 ? one : two;
-        if (js.empty()) continue;
-        // the jobs of two segments first, so that the last blocks to start are short
-        std::stable_sort(js.begin(), js.end(),
-                         [](const FbJobT<float>& a, const FbJobT<float>& b) { return a.nseg > b.nseg; });
-        int maxN = 0;
-        for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
-        g.pipe = g_mixed_gemm.load() == MIXED_GEMM_BF16X6 ? gemm_pipe_kind<float>(js, g.buf_ok) : -1;
-        if (g.pipe >= 0) {
-            int64_t work = 0;
-            for (const auto& j : js) work += (int64_t)j.nseg * j.K * j.Ncol * g.nx;
-            if (work < GEMM_SPLIT_WORK || !split_matrices(js)) g.pipe = -1;
+        for (std::vector<FbJobT<float>>& js : gemm_groups<float>(pass == 0 ? one : two, g, pass + 1)) {
+            if (js.empty()) continue;
+            // the jobs of two segments first, so that the last blocks to start are short
+            std::stable_sort(js.begin(), js.end(),
+                             [](const FbJobT<float>& a, const FbJobT<float>& b) { return a.nseg > b.nseg; });
+            int maxN = 0;
+            for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
+            g.pipe = g_mixed_gemm.load() == MIXED_GEMM_BF16X6 ? gemm_pipe_kind<float>(js, g.buf_ok) : -1;
+            if (g.pipe >= 0) {
+                int64_t work = 0;
+                for (const auto& j : js) work += (int64_t)j.nseg * j.K * j.Ncol * g.nx;
+                if (work < GEMM_SPLIT_WORK || !split_matrices(js)) g.pipe = -1;
+            }
+            const FbJobT<float>* dj =
+                static_cast<const FbJobT<float>*>(device_table(js.data(), js.size() * sizeof(FbJobT<float>)));
+            if (!dj) return ST_ENOMEM;
+            int tile = gemm_choose_tile<FbJobT<float>>(dj, js, maxN, g, pass + 1, 4);
+            if (tile == GT_W4 && pass == 1 && g_mixed_gemm.load() == MIXED_GEMM_BF16X6) tile = GT_W2;
+            CH_TRY(gemm_tile_launch(dj, js.size(), maxN, g, pass + 1, tile));
         }
-        const FbJobT<float>* dj =
-            static_cast<const FbJobT<float>*>(device_table(js.data(), js.size() * sizeof(FbJobT<float>)));
-        if (!dj) return ST_ENOMEM;
-        int tile = gemm_choose_tile<FbJobT<float>>(dj, js, maxN, g, pass + 1, 4);
-        if (tile == GT_W4 && pass == 1 && g_mixed_gemm.load() == MIXED_GEMM_BF16X6) tile = GT_W2;
-        CH_TRY(gemm_tile_launch(dj, js.size(), maxN, g, pass + 1, tile));
     }
     return ST_OK;
 }
