@@ -627,8 +627,10 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
         }
         if (slotted) {
             d = make_int4(br0, bx0, TX, TR);
-            if (a.mask && tid < TR)
-                atomicOr(a.mask + (int64_t)(br0 + tid) * a.words + (grp >> 11), 1u << ((grp >> 6) & 31));
+            // (a narrow tile of one or two modes has more rows than the block threads)
+            if (a.mask)
+                for (int r = tid; r < TR; r += DEP_T)
+                    atomicOr(a.mask + (int64_t)(br0 + r) * a.words + (grp >> 11), 1u << ((grp >> 6) & 31));
         }
     }
     if (tid == 0) a.desc[grp] = d;

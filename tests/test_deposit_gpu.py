@@ -132,6 +132,31 @@ def test_deposit_paths(port, nx, nkr, nko, n, order, precision):
     check(port, coord, half, coord, mom, w, g, out, precision, shift=0.03)
 
 
+# Tiles of two or three node columns and more node rows than a group has
+# threads, with row masks (more than 1024 groups of 256 particles): every row of
+# such a tile must be marked.  "randcell": the order of Species.gen_randcell with
+# one particle a cell (column by column, the radius fastest); "sheet": one column
+# of cells, its particles in random order.
+@pytest.mark.parametrize("nx,nkr,nko,n,order,curr", [(1025, 299, 0, 1024 * 299, "randcell", True),
+                                                     (201, 500, 0, 600000, "sheet", True),
+                                                     (201, 390, 1, 600000, "sheet", False)])
+def test_deposit_tall_tiles(port, nx, nkr, nko, n, order, curr):
+    say(f"case: deposit nx={nx} nkr={nkr} nko={nko} n={n} {order} curr={curr}")
+    g = Grid(nx=nx, nkr=nkr, nko=nko, leftX=-0.05 * nx)
+    r = np.random.default_rng(nkr)
+    if order == "randcell":
+        x = (g.leftX + g.dx * (np.arange(nx - 1)[:, None] + 0.5 * r.uniform(0, 1, (nx - 1, nkr)))).ravel()
+        rr = (g.Rgrid[:-1] + g.dr * 0.5 * (1 + r.uniform(0.02, 1, (nx - 1, nkr)))).ravel()
+    else:
+        x = g.leftX + g.dx * (nx // 2 + r.uniform(0.02, 0.98, n))
+        rr = r.uniform(0.02, g.Rgrid[-1] - 0.02, n)
+    th = r.uniform(0, 2 * np.pi, n)
+    coord = np.vstack([x, rr * np.sin(th), rr * np.cos(th)])
+    mom, w = r.standard_normal((3, n)), r.uniform(0.1, 1.0, n)
+    out = deposit(coord, coord, mom, w, g, curr=curr)
+    check(port, coord, coord, coord, mom, w, g, out, "fp64", curr=curr)
+
+
 @pytest.mark.parametrize("curr,dens", [(True, False), (False, True), (True, True)])
 @pytest.mark.parametrize("ld_extra", [0, 1, 37])
 def test_deposit_push_and_parts(port, curr, dens, ld_extra):
