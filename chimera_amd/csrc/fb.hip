@@ -490,8 +490,10 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm(const FbJob* __restri
 // one lane.  Both stages are swizzled instead of padded (A: blocks of 16 values
 // swapped in odd rows; D: k ^ column), which lets three blocks share a CU.
 // Rows past K hold zeros; x past nx and columns past Ncol compute values that
-// the epilogue does not store (x is clamped to the grid, D reads past the
-// matrix return zero by the buffer's bound).
+// the epilogue does not store.  Every load is inside its array: x, the rows of
+// A and D and the columns of D are clamped in the offsets themselves (the bound
+// of a buffer resource would not do: the instruction's scalar offset is no part
+// of what it checks).
 template <int WN>
 struct GemmPipe {
     static constexpr int BN = 32 * WN, LDA = 2 * GB_X;
@@ -505,11 +507,6 @@ struct GemmPipe {
 
 // Blocks per CU (waves per SIMD) the registers and the LDS allow.
 constexpr int gemm_pipe_occ(int nacc, int wn) { return nacc * wn >= 2 ? 2 : 3; }
-
-// Buffer of n bytes at p: loads past it return zero.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t ch_rsrc_n(const void* p, uint32_t n) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)n, 0x00020000);
-}
 
 // 16-byte store.  Its offset stands whole in the vector register: a store whose
 // scalar offset is a register may still be reading its data when the next
@@ -617,8 +614,11 @@ __global__ void __launch_bounds__(GB_THREADS, gemm_pipe_occ(NACC, WN)) k_fb_gemm
     const uint32_t la0 = seg_lane_a(S0, min(x0 + lane, g.nx - 1), g.nx, g.lda, 0);
     const uint32_t la1 = seg_lane_a(S1, min(x0 + lane, g.nx - 1), g.nx, g.lda, 0);
     const uint32_t ldc = (uint32_t)(S0.ldd * sizeof(double));               // bytes per column of D
-    const uint32_t lcol = (uint32_t)(n0 + (tid >> 4)) * ldc + (uint32_t)(tid & 15) * 8u;
-    const uint32_t dbytes = (uint32_t)(Ncol - 1) * ldc + (uint32_t)K * 8u;
+    // columns n0 + tid/16 + 16i of D: i < nfull are there for all lanes, the others are clamped
+    const int nfull = (Ncol - n0) >> 4;
+    const uint32_t lrow = KR ? 0u : (uint32_t)(tid & 15) * 8u;
+    const uint32_t lcol = (uint32_t)(n0 + (tid >> 4)) * ldc + lrow;
+    const uint32_t lend = (uint32_t)min(n0 + 16 * nfull + (tid >> 4), Ncol - 1) * ldc + lrow;
     double2 ra[NA], rb[A1 ? NA : 1];
     double rd[ND];
     // loads of stage t: A row k = k0 + wave + 4i of x = x0 + lane; D row k0 + tid%16 of columns n0 + tid/16 + 16i
@@ -634,9 +634,12 @@ __global__ void __launch_bounds__(GB_THREADS, gemm_pipe_occ(NACC, WN)) k_fb_gemm
 #pragma unroll
             for (int i = 0; i < NA; i++) rb[i] = ldb_c(rs_b, la, (uint32_t)min(k0 + wave + 4 * i, K - 1) * row, double2{});
         }
-        const __amdgpu_buffer_rsrc_t rs_d = ch_rsrc_n(s ? S1.D : S0.D, dbytes);
+        const __amdgpu_buffer_rsrc_t rs_d = ch_rsrc(s ? S1.D : S0.D);
+        const uint32_t krow = KR ? (uint32_t)min(tid & 15, K - 1 - k0) * 8u : 0u;
 #pragma unroll
-        for (int i = 0; i < ND; i++) rd[i] = ldb_r(rs_d, lcol, (uint32_t)k0 * 8u + (uint32_t)(16 * i) * ldc, double{});
+        for (int i = 0; i < ND; i++)
+            rd[i] = ldb_r(rs_d, (i < nfull ? lcol : lend) + krow,
+                          (uint32_t)k0 * 8u + (i < nfull ? (uint32_t)(16 * i) * ldc : 0u), double{});
     };
     // the loaded values of stage t to LDS buffer B
     auto stash = [&](int t, auto B) __attribute__((always_inline)) {
