@@ -166,8 +166,8 @@ __global__ void __launch_bounds__(GP_T) k_gather_push(const double* __restrict__
 //     from ballots.  A lane takes one (segment, component, node row of the
 //     cell): it sums the particles of the segment on the row's two nodes, all
 //     modes, in FP64 registers and adds the sums to the block's LDS tile (real
-//     planes: Re of mode 0, then Re and Im of each mode) with ds_add_f64.  rho
-//     follows J through the same LDS.
+//     planes: Re of mode 0, then Re and Im of each mode) with ds_add_f64, the
+//     waves one after the other.  rho follows J through the same LDS.
 //  3. The block hands the tile on:
 //      * a tile of at most DEP_SLOT values goes with plain stores, as it is,
 //        into the group's own slot, with a descriptor (first node row, first
@@ -184,10 +184,10 @@ __global__ void __launch_bounds__(GP_T) k_gather_push(const double* __restrict__
 // What bounds it: about equally the 104 bytes per particle in and out of HBM
 // (with the slots 8.9 GB of traffic for 67.0 M electrons at four modes), the
 // segments' arithmetic and their LDS reads and adds; three blocks of a CU share
-// them.  There it takes 2.8 ms, and the combine 0.9; one pass per component over
-// particles re-read from memory (46 GB) took 5.5, with a combine of 1.2.  Mixed
-// precision, 16.7 M at three modes: 0.75 + 0.11 ms, before 1.24 + 0.13 and 70 us
-// to sort the slots.  (Loading the next group during the deposit of one, a
+// them.  There it takes 3.1 ms (2.8 without the fixed order of the adds), and the
+// combine 0.9; one pass per component over particles re-read from memory (46 GB)
+// took 5.5, with a combine of 1.2.  Mixed precision, 16.7 M at three modes: 0.82 +
+// 0.11 ms, before 1.24 + 0.13 and 70 us to sort the slots.  (Loading the next group during the deposit of one, a
 // block taking several, changed nothing: the other blocks already hide it.)
 
 template <typename RT>
@@ -347,20 +347,36 @@ __device__ __forceinline__ int dep_segments(DepWave<PPL>& L, const uint32_t (&ke
 
 // The wave's segments into components c0..c0+NCP-1 (charges L.q[c0..]): to the
 // tile (pns values per component: planes of nn nodes, rows of TX; key = node of
-// the cell's lower corner), or, untiled, straight to the grid (key = node offset in a mode plane).  The
-// lanes of one ds_add_f64 add to different nodes.  (With all four corners in a
-// lane the segments had to be cut shorter to fill the lanes, and several of one
-// cell collided on every add.)
+// the cell's lower corner), or, untiled, straight to the grid (key = node offset
+// in a mode plane).  The lanes of one ds_add_f64 mostly add to different nodes.
+// (With all four corners in a lane the segments had to be cut shorter to fill
+// the lanes, and several of one cell collided on every add.)
+//
+// The waves add to the tile in turn, a round of 64 lanes each, so that its sums
+// have the same order in every call: a barrier between two turns, and as many
+// rounds as the block's wave with the most segments has (nsegs: the number of
+// each, exchanged at the first barrier).  No barrier after the last turn.  On
+// 67.0 M electrons at four modes, 10 steps after a sort, 4.13 ms with the combine; unordered
+// 3.82, but with other last bits in every call.  (Tried: the even waves and then
+// the odd ones where their boxes allow it, 4.11; a wave waiting for the waves
+// that share nodes with it alone, by counters in LDS, 4.05; the odd waves
+// keeping the sums of shared nodes in registers until the others are done, 4.25.)
 template <int NMOD, int NCP, int PPL, typename R>
-__device__ __forceinline__ void dep_pass(DepWave<PPL>& L, int nseg, int c0, bool tiled, double* tile, int pns, int nn,
-                                         int TX, cplx_t<R>* grid, int64_t sr, int64_t sm, int64_t sl) {
+__device__ __forceinline__ void dep_pass(DepWave<PPL>& L, int wv, int nseg, int* nsegs, int c0, bool tiled,
+                                         double* tile, int pns, int nn, int TX, cplx_t<R>* grid, int64_t sr, int64_t sm,
+                                         int64_t sl) {
     constexpr int PL = 2 * NMOD - 1;
-    for (int t = threadIdx.x & 63; t < nseg * (2 * NCP); t += 64) {
-        const int sg = t / (2 * NCP), rem = t - sg * (2 * NCP), c = rem >> 1;
+    const int nt = nseg * (2 * NCP);
+    int rounds = (nt + 63) >> 6;          // of this wave; at least one
+    if (tiled && (threadIdx.x & 63) == 0) nsegs[wv] = nseg;
+    for (int r = 0, t = threadIdx.x & 63; r < rounds; r++, t += 64) {
+        const bool in = t < nt;
+        const int sg = in ? t / (2 * NCP) : 0, rem = in ? t - sg * (2 * NCP) : 0, c = rem >> 1;
         const bool up = rem & 1;
-        const int pb = L.seg[sg], pe = L.seg[sg + 1];
+        const int pb = L.seg[sg], pe1 = L.seg[sg + 1];
         const uint32_t key = L.cell[pb];
-        if (key == DEP_SKIP) continue;
+        const bool on = in && key != DEP_SKIP;
+        const int pe = on ? pe1 : pb;
         const double* q = L.q[c0 + c];
         double acc[PL][2];
 #pragma unroll
@@ -384,11 +400,23 @@ __device__ __forceinline__ void dep_pass(DepWave<PPL>& L, int nseg, int c0, bool
         }
         if (tiled) {
             double* tp = tile + c * pns + key + (up ? TX : 0);
+            for (int w = 0; w < DEP_WAVES; w++) {
+                if (w == wv && on) {
 #pragma unroll
-            for (int i = 0; i < PL; i++)
+                    for (int i = 0; i < PL; i++)
 #pragma unroll
-                for (int k = 0; k < 2; k++) lds_add(tp + i * nn + k, acc[i][k]);
-        } else {
+                        for (int k = 0; k < 2; k++) lds_add(tp + i * nn + k, acc[i][k]);
+                }
+                if (w + 1 < DEP_WAVES) __syncthreads();
+            }
+            if (r == 0) {
+                int n = 0;
+#pragma unroll
+                for (int i = 0; i < DEP_WAVES; i++) n = max(n, nsegs[i]);
+                rounds = __builtin_amdgcn_readfirstlane((n * (2 * NCP) + 63) >> 6);
+            }
+            if (r + 1 < rounds) __syncthreads();
+        } else if (on) {
 #pragma unroll
             for (int m = 0; m < NMOD; m++)
 #pragma unroll
@@ -442,7 +470,8 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
     __shared__ DepWave<PPL> wl[DEP_WAVES];
     __shared__ __align__(16) double tile[DEP_POOL];
     __shared__ int red[DEP_WAVES][4];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    __shared__ int nsegs[2][DEP_WAVES];         // of J, of rho
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const GridGeom gJ = frame_geom(a.gJ), gR = frame_geom(a.gR);
     const int64_t ld = a.ld;
     const bool doJ = a.J != nullptr, doR = a.R != nullptr;
@@ -583,7 +612,7 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
             keys(okJ, ixJ, irJ, key);
             const int nseg = dep_segments<PPL, 3>(L, key);
             if (per != 1) {
-                dep_pass<NMOD, 3, PPL, R>(L, nseg, 0, tiled, tile, pns, nn, TX, a.J, sr, sm, sl);
+                dep_pass<NMOD, 3, PPL, R>(L, wv, nseg, nsegs[0], 0, tiled, tile, pns, nn, TX, a.J, sr, sm, sl);
                 if (per == 3) {
                     __syncthreads();
                     dep_writeout<NMOD, R>(tile, 3, pns, nn, TX, slot, a.J + corner, sr, sm);
@@ -592,7 +621,7 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
             } else {
 #pragma unroll 1
                 for (int c = 0; c < 3; c++) {
-                    dep_pass<NMOD, 1, PPL, R>(L, nseg, c, true, tile, pns, nn, TX, a.J, sr, sm, sl);
+                    dep_pass<NMOD, 1, PPL, R>(L, wv, nseg, nsegs[0], c, true, tile, pns, nn, TX, a.J, sr, sm, sl);
                     __syncthreads();
                     dep_writeout<NMOD, R>(tile, 1, pns, nn, TX, slot ? slot + c * pns : nullptr,
                                           a.J + c * sl + corner, sr, sm);
@@ -612,7 +641,8 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
                 }
             keys(okR, ixR, irR, key);
             const int nseg = dep_segments<PPL, 1>(L, key);
-            dep_pass<NMOD, 1, PPL, R>(L, nseg, 0, tiled, tile + (per == 4 ? rho0 : 0), pns, nn, TX, a.R, sr, sm, sl);
+            dep_pass<NMOD, 1, PPL, R>(L, wv, nseg, nsegs[1], 0, tiled, tile + (per == 4 ? rho0 : 0), pns, nn, TX, a.R, sr,
+                                      sm, sl);
             if (tiled) {
                 __syncthreads();
                 if (per != 4) {

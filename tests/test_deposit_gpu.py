@@ -191,3 +191,21 @@ def test_deposit_skips_and_lost_particles(port):
     assert rel_max(out[2], ref[2]) < 1e-13 and rel_max(out[3], ref[3]) < 1e-13
     none = deposit(bad, bad, np.ones((3, 7)), np.ones(7), g)
     assert not np.any(none[2]) and not np.any(none[3])
+
+
+# groups that all hand their tile on in a slot: every way the components share
+# the LDS, both group sizes, one and several rounds of segments a wave
+@pytest.mark.parametrize("nx,nkr,nko,n,order,precision", [
+    (13, 6, 1, 20001, "shuffled", "fp64"), (13, 6, 3, 20001, "shuffled", "fp64"), (65, 16, 2, 300001, "sorted", "fp64"),
+    (65, 16, 2, 300001, "sorted", "mixed"), (33, 16, 1, 40000, "sorted", "fp64"), (13, 6, 4, 300000, "sorted", "fp64")])
+def test_deposit_same_bits(nx, nkr, nko, n, order, precision):
+    """The sums of slotted tiles have one order: the same bits from call to call."""
+    say(f"case: deposit bits nx={nx} nkr={nkr} nko={nko} n={n} {order} {precision}")
+    g = Grid(nx=nx, nkr=nkr, nko=nko, leftX=-0.05 * nx)
+    coord, mom, w = particles(g, n, seed=n)
+    if order == "sorted":
+        coord, mom, w = cell_sorted(coord, mom, w, g)
+    first = deposit(coord, coord, mom, w, g, precision)
+    for _ in range(5):
+        again = deposit(coord, coord, mom, w, g, precision)
+        assert all(np.array_equal(a, b) for a, b in zip(first, again))
