@@ -90,7 +90,9 @@ class Stage {
 // Scratch device memory of the current context, grown on demand and reused
 // across calls on its stream (the stream orders every use).  It cannot grow
 // while the context captures a step or while graphs captured on it are alive.
-void* scratch(int slot, size_t bytes);
+// Null where it cannot grow; with `optional` (the caller does without) no error
+// text is left.
+void* scratch(int slot, size_t bytes, bool optional = false);
 // Byte fill of device memory by a kernel on the library stream (no hipMemsetAsync,
 // so that a captured graph replays it correctly).
 int32_t fill_bytes(void* p, int value, size_t bytes);

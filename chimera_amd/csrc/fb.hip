@@ -1011,7 +1011,7 @@ static int gemm_choose_tile(const J* dj, const std::vector<J>& js, int maxN, con
     if (capturing()) return rule;
     // the job table with every output in one scratch buffer of ldo * maxN elements
     std::vector<J> tj(js);
-    void* sink = scratch(20, (size_t)g.ldo * maxN * 2 * rbytes);
+    void* sink = scratch(20, (size_t)g.ldo * maxN * 2 * rbytes, true);
     if (!sink) return rule;
     for (auto& j : tj)
         for (int o = 0; o < j.nout; o++) j.out[o].p = static_cast<decltype(j.out[o].p)>(sink);
@@ -1834,8 +1834,9 @@ static int32_t launch_gemm_bf16_pipe(const FbJobT<float>* dj, size_t njobs, int 
 }
 
 // The pieces of every matrix of the jobs into scratch slot 17, and Seg::ds set;
-// false where the scratch has no room for them.
-static bool split_matrices(std::vector<FbJobT<float>>& js) {
+// done = false, and nothing changed, where the scratch has no room for them.
+static int32_t split_matrices(std::vector<FbJobT<float>>& js, bool& done) {
+    done = false;
     typedef std::tuple<const float*, int64_t, int, int> Key;
     std::map<Key, int64_t> at;
     int64_t bytes = 0, most = 0;
@@ -1847,9 +1848,9 @@ static bool split_matrices(std::vector<FbJobT<float>>& js) {
             most = b > most ? b : most;
             bytes += b;
         }
-    if (most >= (int64_t)1 << 31) return false;
-    char* const p = static_cast<char*>(scratch(17, (size_t)bytes));
-    if (!p) return false;
+    if (most >= (int64_t)1 << 31) return ST_OK;
+    char* const p = static_cast<char*>(scratch(17, (size_t)bytes, true));
+    if (!p) return ST_OK;
     std::vector<SplitMat> mats;
     for (const auto& kv : at) {
         SplitMat m;
@@ -1866,10 +1867,12 @@ static bool split_matrices(std::vector<FbJobT<float>>& js) {
         for (int q = 0; q < j.nseg; q++)
             j.seg[q].ds = p + at[Key(j.seg[q].D, j.seg[q].ldd, j.K, j.Ncol)];
     const SplitMat* dm = static_cast<const SplitMat*>(device_table(mats.data(), mats.size() * sizeof(SplitMat)));
-    if (!dm) return false;
+    if (!dm) return ST_ENOMEM;
     const dim3 grid((unsigned)((most / 192 * 4 + 255) / 256), (unsigned)mats.size());
     hipLaunchKernelGGL(k_split_d, grid, 256, 0, stream(), dm);
-    return hipGetLastError() == hipSuccess;
+    CH_LAUNCH_CHECK("k_split_d");
+    done = true;
+    return ST_OK;
 }
 
 template <int NACC, int WN, int GX>
@@ -1920,7 +1923,9 @@ int32_t launch_fb_gemm<float>(const std::vector<FbJobT<float>>& jobs, const FbGe
             if (g.pipe >= 0) {
                 int64_t work = 0;
                 for (const auto& j : js) work += (int64_t)j.nseg * j.K * j.Ncol * g.nx;
-                if (work < GEMM_SPLIT_WORK || !split_matrices(js)) g.pipe = -1;
+                bool split = false;
+                if (work >= GEMM_SPLIT_WORK) CH_TRY(split_matrices(js, split));
+                if (!split) g.pipe = -1;
             }
             const FbJobT<float>* dj =
                 static_cast<const FbJobT<float>*>(device_table(js.data(), js.size() * sizeof(FbJobT<float>)));

@@ -104,6 +104,7 @@ int32_t fail(int32_t code, const char* fmt, ...) {
 }
 
 int32_t hip_fail(hipError_t e, const char* what, const char* file, int line) {
+    (void)hipGetLastError();    // reported here: the next launch check is not to find it again
     set_error("%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
     return e == hipErrorOutOfMemory ? ST_ENOMEM : ST_EHIP;
 }
@@ -111,6 +112,15 @@ int32_t hip_fail(hipError_t e, const char* what, const char* file, int line) {
 hipStream_t stream() { return cur().stream; }
 void set_stream(hipStream_t s) { cur().stream = s; }
 bool capturing() { return cur().capturing; }
+
+// hipMalloc, or null: the runtime keeps a failure as its last error until it is
+// read, and the next launch check would take it for that launch's.
+static void* device_alloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
 
 bool is_device_ptr(const void* p) {
     if (p == nullptr) return false;
@@ -171,20 +181,22 @@ Stage::~Stage() {
     }
 }
 
-void* scratch(int slot, size_t bytes) {
+void* scratch(int slot, size_t bytes, bool optional) {
     std::lock_guard<std::mutex> lk(g_mu);
     Context& c = cur();
     ScratchSlot& s = c.scratch[slot];
     if (s.bytes >= bytes && s.p) return s.p;
     if (c.capturing) {
-        set_error("scratch slot %d must grow to %zu bytes inside a captured step: run the step once before "
-                  "capturing it", slot, bytes);
+        if (!optional)
+            set_error("scratch slot %d must grow to %zu bytes inside a captured step: run the step once before "
+                      "capturing it", slot, bytes);
         return nullptr;
     }
     if (s.p) {
         if (c.graphs > 0) {
-            set_error("scratch slot %d must grow to %zu bytes while graphs captured on this context still use it",
-                      slot, bytes);
+            if (!optional)
+                set_error("scratch slot %d must grow to %zu bytes while graphs captured on this context still use it",
+                          slot, bytes);
             return nullptr;
         }
         (void)hipStreamSynchronize(c.stream);
@@ -193,9 +205,9 @@ void* scratch(int slot, size_t bytes) {
         s.bytes = 0;
     }
     size_t want = bytes < 256 ? 256 : bytes;
-    if (hipMalloc(&s.p, want) != hipSuccess) {
-        s.p = nullptr;
-        set_error("hipMalloc of %zu scratch bytes failed", want);
+    s.p = device_alloc(want);
+    if (!s.p) {
+        if (!optional) set_error("hipMalloc of %zu scratch bytes failed", want);
         return nullptr;
     }
     s.bytes = want;
@@ -218,8 +230,8 @@ const void* device_table(const void* host, size_t bytes) {
         for (auto& kv : c.tables) (void)hipFree(kv.second);
         c.tables.clear();
     }
-    void* d = nullptr;
-    if (hipMalloc(&d, bytes) != hipSuccess) {
+    void* d = device_alloc(bytes);
+    if (!d) {
         set_error("hipMalloc of a %zu-byte table failed", bytes);
         return nullptr;
     }
@@ -243,8 +255,8 @@ const void* shared_table(const void* host, size_t bytes) {
                   "capturing it", bytes);
         return nullptr;
     }
-    void* d = nullptr;
-    if (hipMalloc(&d, bytes) != hipSuccess) {
+    void* d = device_alloc(bytes);
+    if (!d) {
         set_error("hipMalloc of a %zu-byte shared table failed", bytes);
         return nullptr;
     }

@@ -44,3 +44,29 @@ def test_edges(gpu, port, nkx, nkr, nko, name):
     assert e < TOL32
     for _ in range(3):
         assert np.array_equal(_c8(OPS[name], out.copy(order="F"), inp, Dp, Dm, kx, nko), first)
+
+
+def _operands(nkx, nkr, nko, seed):
+    """Device operands of one large mixed divergence and a function that runs it."""
+    from chimera_amd.device import DeviceArray, call
+    r = rng(seed)
+    d = lambda a, t: DeviceArray.from_numpy(a, t)                                    # noqa: E731
+    a = [d(C(r, nkx, nkr, nko + 1, 3), np.complex64), d(F(r, nkr, nkr, nko + 2), np.float32),
+         d(F(r, nkr, nkr, nko + 2), np.float32), DeviceArray.from_numpy(2 * np.pi * np.fft.fftfreq(nkx, 1.0))]
+    out = DeviceArray((nkx, nkr, nko + 1), np.complex64)
+    return out, lambda: call("chimera_fb_op_c8", OPS["div"], out.ptr, *(x.ptr for x in a), nkx, nkr, nko)
+
+
+def _capture(run):
+    import ctypes
+    from chimera_amd._lib import DEVICE_LOCK, check, lib
+    with DEVICE_LOCK:
+        check("chimera_capture_begin", lib().chimera_capture_begin())
+        try:
+            run()
+        except Exception:
+            lib().chimera_capture_abort()
+            raise
+        h = ctypes.c_void_p(0)
+        check("chimera_capture_end", lib().chimera_capture_end(ctypes.byref(h)))
+    return h.value
