@@ -1546,7 +1546,7 @@ struct GemmPipeBf {
 };
 struct SplitMat {
     const float* D;
-    uint16_t* out;
+    int64_t out;            // bytes from the scratch of the pieces
     int64_t ldd;
     int K, Ncol, npad;
 };
@@ -1554,7 +1554,7 @@ constexpr int gbb_npad(int Ncol) { return (Ncol + 127) / 128 * 128; }
 constexpr int64_t gbb_bytes(int K, int Ncol) { return (int64_t)((K + GBB_K - 1) / GBB_K) * 3 * gbb_npad(Ncol) * 64; }
 
 // Pieces of the matrices of a launch: thread = 8 k of one column.
-__global__ void __launch_bounds__(256) k_split_d(const SplitMat* __restrict__ mats) {
+__global__ void __launch_bounds__(256) k_split_d(const SplitMat* __restrict__ mats, char* __restrict__ pieces) {
     const SplitMat m = mats[blockIdx.y];
     const int stages = (m.K + GBB_K - 1) / GBB_K;
     const int64_t n = (int64_t)stages * m.npad * 4;
@@ -1567,7 +1567,7 @@ __global__ void __launch_bounds__(256) k_split_d(const SplitMat* __restrict__ ma
             const float v = col < m.Ncol && k + q < m.K ? m.D[k + q + m.ldd * col] : 0.f;
             split3_bf16(v, h[q], md[q], l[q]);
         }
-        uint16_t* const o = m.out + ((int64_t)st * 3 * m.npad + col) * GBB_K + part * 8;
+        uint16_t* const o = reinterpret_cast<uint16_t*>(pieces + m.out) + ((int64_t)st * 3 * m.npad + col) * GBB_K + part * 8;
         const int64_t pp = (int64_t)m.npad * GBB_K;
         lds_store_bf16<8>(o, h);
         lds_store_bf16<8>(o + pp, md);
@@ -1702,7 +1702,7 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm_bf16_pipe(const FbJob
     };
     auto fetch_d = [&](int t) __attribute__((always_inline)) {
         const bool s = t >= sps;
-        const __amdgpu_buffer_rsrc_t rs_d = ch_rsrc(s ? S1.ds : S0.ds);
+        const __amdgpu_buffer_rsrc_t rs_d = ch_rsrc(g.split + (s ? S1.ds : S0.ds));
         const uint32_t so = (uint32_t)(s ? t - sps : t) * 3u * dpiece;
 #pragma unroll
         for (int p = 0; p < 3; p++)
@@ -1834,9 +1834,12 @@ static int32_t launch_gemm_bf16_pipe(const FbJobT<float>* dj, size_t njobs, int 
 }
 
 // The pieces of every matrix of the jobs into scratch slot 17, and Seg::ds set;
-// done = false, and nothing changed, where the scratch has no room for them.
-static int32_t split_matrices(std::vector<FbJobT<float>>& js, bool& done) {
-    done = false;
+// pieces = null, and nothing changed, where the scratch has no room for them.  The
+// device tables hold offsets, not addresses: they stay the same when another
+// operator of the step makes the scratch grow, so that one eager pass uploads all
+// that a capture of the step reads.
+static int32_t split_matrices(std::vector<FbJobT<float>>& js, const char*& pieces) {
+    pieces = nullptr;
     typedef std::tuple<const float*, int64_t, int, int> Key;
     std::map<Key, int64_t> at;
     int64_t bytes = 0, most = 0;
@@ -1856,7 +1859,7 @@ static int32_t split_matrices(std::vector<FbJobT<float>>& js, bool& done) {
         SplitMat m;
         memset(&m, 0, sizeof m);
         m.D = std::get<0>(kv.first);
-        m.out = reinterpret_cast<uint16_t*>(p + kv.second);
+        m.out = kv.second;
         m.ldd = std::get<1>(kv.first);
         m.K = std::get<2>(kv.first);
         m.Ncol = std::get<3>(kv.first);
@@ -1865,13 +1868,13 @@ static int32_t split_matrices(std::vector<FbJobT<float>>& js, bool& done) {
     }
     for (auto& j : js)
         for (int q = 0; q < j.nseg; q++)
-            j.seg[q].ds = p + at[Key(j.seg[q].D, j.seg[q].ldd, j.K, j.Ncol)];
+            j.seg[q].ds = at[Key(j.seg[q].D, j.seg[q].ldd, j.K, j.Ncol)];
     const SplitMat* dm = static_cast<const SplitMat*>(device_table(mats.data(), mats.size() * sizeof(SplitMat)));
     if (!dm) return ST_ENOMEM;
     const dim3 grid((unsigned)((most / 192 * 4 + 255) / 256), (unsigned)mats.size());
-    hipLaunchKernelGGL(k_split_d, grid, 256, 0, stream(), dm);
+    hipLaunchKernelGGL(k_split_d, grid, 256, 0, stream(), dm, p);
     CH_LAUNCH_CHECK("k_split_d");
-    done = true;
+    pieces = p;
     return ST_OK;
 }
 
@@ -1923,9 +1926,9 @@ int32_t launch_fb_gemm<float>(const std::vector<FbJobT<float>>& jobs, const FbGe
             if (g.pipe >= 0) {
                 int64_t work = 0;
                 for (const auto& j : js) work += (int64_t)j.nseg * j.K * j.Ncol * g.nx;
-                bool split = false;
-                if (work >= GEMM_SPLIT_WORK) CH_TRY(split_matrices(js, split));
-                if (!split) g.pipe = -1;
+                g.split = nullptr;
+                if (work >= GEMM_SPLIT_WORK) CH_TRY(split_matrices(js, g.split));
+                if (!g.split) g.pipe = -1;
             }
             const FbJobT<float>* dj =
                 static_cast<const FbJobT<float>*>(device_table(js.data(), js.size() * sizeof(FbJobT<float>)));
@@ -1949,7 +1952,7 @@ static FbSegT<R> seg(const cplx_t<R>* a0, double2 c0, const cplx_t<R>* a1, doubl
     s.c0 = c0;
     s.c1 = c1;
     s.D = D;
-    s.ds = nullptr;
+    s.ds = 0;
     s.ldd = ldd;
     s.refl = refl;
     s.acc = acc;

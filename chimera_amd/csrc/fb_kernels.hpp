@@ -57,7 +57,7 @@ struct FbSegT {
     const C* a1;
     double2 c0, c1;
     const R* D;
-    const void* ds;                // set by launch_fb_gemm<float>: D in BF16 pieces (k_split_d)
+    int64_t ds;                    // set by launch_fb_gemm<float>: D in BF16 pieces (k_split_d), bytes from FbGemmArgs::split
     int64_t ldd;
     int refl;
     int acc;
@@ -94,6 +94,7 @@ struct FbGemmArgs {
     double dt_inv;
     int buf_ok;            // set by launch_fb_gemm: every operand offset fits the 31 bits of a buffer load
     int pipe;              // set by launch_fb_gemm: kind of the segments (gemm_pipe_kind)
+    const char* split;     // set by launch_fb_gemm<float>: the matrices in BF16 pieces
 };
 
 enum { FB_ROT = 0, FB_GRAD = 1, FB_DIV = 2, FB_GRADDIV = 3 };

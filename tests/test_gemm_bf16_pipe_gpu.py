@@ -70,3 +70,24 @@ def _capture(run):
         h = ctypes.c_void_p(0)
         check("chimera_capture_end", lib().chimera_capture_end(ctypes.byref(h)))
     return h.value
+
+
+def test_split_captured_after_one_pass(gpu):
+    """A step whose second operator needs more room for its matrices than the
+    first is recorded after one eager pass, and every replay gives its bits."""
+    from chimera_amd._lib import check, lib
+    from chimera_amd.batch import Context
+    say("case: two large mixed operators, one eager pass, capture, replays")
+    with Context() as ctx:
+        (o1, f1), (o2, f2) = _operands(4100, 300, 1, 31), _operands(1030, 544, 1, 32)
+        f1(), f2()
+        ref = o1.numpy(), o2.numpy()
+        g = _capture(lambda: (f1(), f2()))
+        for _ in range(3):
+            o1.write(0, np.zeros(o1.size, np.complex64))
+            o2.write(0, np.zeros(o2.size, np.complex64))
+            check("chimera_graph_launch", lib().chimera_graph_launch(g))
+            ctx.synchronize()
+            assert np.array_equal(o1.numpy(), ref[0]) and np.array_equal(o2.numpy(), ref[1])
+        check("chimera_graph_destroy", lib().chimera_graph_destroy(g))
+    ctx.close()
