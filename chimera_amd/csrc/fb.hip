@@ -579,22 +579,57 @@ __device__ __forceinline__ void gemm_epilogue_full(const FbJob& J, const FbGemmA
     }
 }
 
+// The tiles of a pipeline launch: 64 complex x by one column tile of one job.
+// Every XCD (workgroup id mod 8) takes an eighth of the x tiles, for all jobs
+// alike; the column tiles of one x tile, which read the same A, are next to each
+// other there.  The nxt % 8 x tiles that are left over come first and go round
+// the XCDs one by one: given whole to some of the XCDs they left the others idle
+// (forward transform at 256 x 1024, four modes, 400 us with four XCDs at work,
+// 218 so; Poisson correction there 612 and 371, at 576 x 512 345 and 263; multiples
+// of 512 are as before).
+struct PipeGrid {
+    int nyt, q, r, nrem;         // column tiles, nxt / 8, nxt % 8, blocks of the r tiles
+    unsigned blocks;
+};
+static PipeGrid pipe_grid(int nx, int maxN, int cols, size_t njobs) {
+    const int nxt = (nx + GB_X - 1) / GB_X;
+    PipeGrid p;
+    p.nyt = (maxN + cols - 1) / cols;
+    p.q = nxt / 8, p.r = nxt % 8;
+    p.nrem = (int)(p.r * p.nyt * njobs);
+    p.blocks = (unsigned)((size_t)nxt * p.nyt * njobs);
+    return p;
+}
+__device__ __forceinline__ void pipe_tile(const PipeGrid& p, int& xt, int& yt, int& job) {
+    int id = blockIdx.x;
+    if (id < p.nrem) {
+        yt = id % p.nyt;
+        id /= p.nyt;
+        xt = 8 * p.q + id % p.r;
+        job = id / p.r;
+    } else {
+        id -= p.nrem;
+        xt = id & 7;
+        id >>= 3;
+        yt = id % p.nyt;
+        id /= p.nyt;
+        xt += 8 * (id % p.q);
+        job = id / p.q;
+    }
+}
+
 // KR: some K of the launch is no multiple of GB_K.
 template <int NACC, int WN, bool A1, bool KR>
 __global__ void __launch_bounds__(GB_THREADS, gemm_pipe_occ(NACC, WN)) k_fb_gemm_pipe(const FbJob* __restrict__ jobs,
-                                                                                      FbGemmArgs g, int nx8, int nyt) {
+                                                                                      FbGemmArgs g, PipeGrid pg) {
     typedef GemmPipe<WN> G;
     constexpr int NI = 4, BN = G::BN, NA = G::NA, ND = G::ND;
-    // every XCD (workgroup id mod 8) takes an eighth of the x tiles, for all jobs
-    // alike; the column tiles of one x tile, which read the same A, are next to
-    // each other there
-    int id = blockIdx.x >> 3;
-    const int yt = id % nyt;
-    id /= nyt;
-    const int n0 = yt * BN, x0 = ((id % nx8) * 8 + (blockIdx.x & 7)) * GB_X;
-    const FbJob& J = jobs[id / nx8];
+    int xt, yt, job;
+    pipe_tile(pg, xt, yt, job);
+    const int n0 = yt * BN, x0 = xt * GB_X;
+    const FbJob& J = jobs[job];
     const int Ncol = J.Ncol, K = J.K, nseg = J.nseg;
-    if (n0 >= Ncol || x0 >= g.nx) return;
+    if (n0 >= Ncol) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave & 1, wc = wave >> 1;
 
@@ -763,9 +798,8 @@ static int32_t launch_gemm_pipe_k(const FbJob* dj, size_t njobs, int maxN, const
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         attr = true;
     }
-    const int nx8 = (g.nx + 8 * GB_X - 1) / (8 * GB_X), nyt = (maxN + 32 * WN - 1) / (32 * WN);
-    const unsigned grid = (unsigned)((size_t)nx8 * 8 * nyt * njobs);
-    hipLaunchKernelGGL((k_fb_gemm_pipe<NACC, WN, A1, KR>), grid, GB_THREADS, lds, stream(), dj, g, nx8, nyt);
+    const PipeGrid pg = pipe_grid(g.nx, maxN, 32 * WN, njobs);
+    hipLaunchKernelGGL((k_fb_gemm_pipe<NACC, WN, A1, KR>), pg.blocks, GB_THREADS, lds, stream(), dj, g, pg);
     CH_LAUNCH_CHECK("k_fb_gemm_pipe");
     return ST_OK;
 }
@@ -1649,18 +1683,16 @@ __device__ __forceinline__ void gemm_epilogue_full_f(const FbJobT<float>& J, con
 // KR: some K of the launch is no multiple of GBB_K.
 template <int NACC, int WN, bool A1, bool KR>
 __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm_bf16_pipe(const FbJobT<float>* __restrict__ jobs,
-                                                                     FbGemmArgs g, int nx8, int nyt) {
+                                                                     FbGemmArgs g, PipeGrid pg) {
     typedef GemmPipeBf<WN> G;
     typedef FbSegT<float> Seg;
     constexpr int NI = 4, BN = G::BN, KA = G::KA, ND = G::ND;
-    // blocks to tiles as in k_fb_gemm_pipe
-    int id = blockIdx.x >> 3;
-    const int yt = id % nyt;
-    id /= nyt;
-    const int n0 = yt * BN, x0 = ((id % nx8) * 8 + (blockIdx.x & 7)) * GB_X;
-    const FbJobT<float>& J = jobs[id / nx8];
+    int xt, yt, job;
+    pipe_tile(pg, xt, yt, job);
+    const int n0 = yt * BN, x0 = xt * GB_X;
+    const FbJobT<float>& J = jobs[job];
     const int Ncol = J.Ncol, K = J.K, nseg = J.nseg;
-    if (n0 >= Ncol || x0 >= g.nx) return;
+    if (n0 >= Ncol) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave & 1, wc = wave >> 1;
 
@@ -1816,9 +1848,8 @@ static int32_t launch_gemm_bf16_pipe_k(const FbJobT<float>* dj, size_t njobs, in
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         attr = true;
     }
-    const int nx8 = (g.nx + 8 * GB_X - 1) / (8 * GB_X), nyt = (maxN + 32 * WN - 1) / (32 * WN);
-    const unsigned grid = (unsigned)((size_t)nx8 * 8 * nyt * njobs);
-    hipLaunchKernelGGL((k_fb_gemm_bf16_pipe<NACC, WN, A1, KR>), grid, GB_THREADS, lds, stream(), dj, g, nx8, nyt);
+    const PipeGrid pg = pipe_grid(g.nx, maxN, 32 * WN, njobs);
+    hipLaunchKernelGGL((k_fb_gemm_bf16_pipe<NACC, WN, A1, KR>), pg.blocks, GB_THREADS, lds, stream(), dj, g, pg);
     CH_LAUNCH_CHECK("k_fb_gemm_bf16_pipe");
     return ST_OK;
 }

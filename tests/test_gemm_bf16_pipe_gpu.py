@@ -18,12 +18,15 @@ pytestmark = pytest.mark.gpu
 
 # 8190 x 160: 128-column tiles with 32 columns left, two x of the last tile
 # missing; 4100 x 300: K remainder 12; 1030 x 544: 64-column tiles; 520 x 520:
-# 32-column tiles, K remainder 8
+# 32-column tiles, K remainder 8; 190 x 1024: three x tiles, fewer than XCDs;
+# 830 x 544: 13, five more than XCDs
 @pytest.mark.timeout(900)
 @pytest.mark.parametrize("nkx,nkr,nko,name", [(8190, 160, 1, "div"), (8190, 160, 1, "rot"), (4100, 300, 1, "grad"),
                                               (4100, 300, 1, "graddiv"), (1030, 544, 1, "div"),
                                               (1030, 544, 1, "grad"), (520, 520, 2, "graddiv"),
-                                              (520, 520, 2, "rot")])
+                                              (520, 520, 2, "rot"), (190, 1024, 2, "rot"),
+                                              (190, 1024, 2, "div"), (830, 544, 1, "rot"),
+                                              (830, 544, 1, "graddiv")])
 def test_edges(gpu, port, nkx, nkr, nko, name):
     say(f"case: fb_{name} nkx={nkx} nkr={nkr} nko={nko}")
     r = rng(9000 + nkx + nkr)
