@@ -1088,25 +1088,52 @@ static int gemm_choose_tile(const J* dj, const std::vector<J>& js, int maxN, con
     return best;
 }
 
-// The launches of a job list: one, or one per kind where the list mixes the two
-// kinds and is large enough for the 64-complex-x tiles, whose pipeline takes one
-// kind (the curl's list of one accumulator: at 8192 x 512, four modes, 2.33 ms in
-// one launch of 32-complex-x tiles).
+// The split of the matrices is a launch more: for launches of at least 2^29
+// products of a real by a complex value (forward transform, matrices split in
+// the kernel and once per call, microseconds of the whole call, FFT included:
+// 1024 x 128 x 2 modes 29 and 31, 2048 x 128 x 2 39 and 40, 1024 x 256 x 3, 6e8
+// products, 66 and 54, 1024 x 500 x 2 114 and 77; Poisson correction 2048 x 128 x 2
+// 49 and 55, 4096 x 128 x 3 101 and 70).
+constexpr int64_t GEMM_SPLIT_WORK = (int64_t)1 << 29;
+
+template <typename J>
+static int max_cols(const std::vector<J>& js) {
+    int n = 0;
+    for (const auto& j : js) n = j.Ncol > n ? j.Ncol : n;
+    return n;
+}
+
+// Whether a launch of these jobs goes to the pipeline of its element type: one
+// kind, tiles of 64 complex x, and in mixed precision the split-BF16 form and
+// enough work to split the matrices for.
+template <typename R>
+static bool gemm_piped(const std::vector<FbJobT<R>>& js, const FbGemmArgs& g, int nacc) {
+    if (js.empty() || gemm_pipe_kind<R>(js, g.buf_ok) < 0) return false;
+    if (gemm_tile(g.nx, max_cols(js), js.size(), sizeof(R) == 4 || nacc == 1) >= GT_H) return false;
+    if (sizeof(R) == 8) return true;
+    int64_t work = 0;
+    for (const auto& j : js) work += (int64_t)j.nseg * j.K * j.Ncol * g.nx;
+    return g_mixed_gemm.load() == MIXED_GEMM_BF16X6 && work >= GEMM_SPLIT_WORK;
+}
+
+// The launches of a job list: one, or one per kind of segments where the list
+// mixes the two and a pipeline, which takes one kind, takes at least one of them
+// (the curl's list of one accumulator: in FP64 at 8192 x 512, four modes, 2.33 ms
+// in one launch of 32-complex-x tiles, 1.2 in two).  Where none goes to a pipeline
+// two launches only cost: mixed, four modes, 1088 x 256 115 us in one and 135 in two,
+// FP32 form 2048 x 128 54 and 60; with one of the two in the pipeline, 1600 x 256
+// 157 and 129.
 template <typename R>
 static std::vector<std::vector<FbJobT<R>>> gemm_groups(const std::vector<FbJobT<R>>& js, const FbGemmArgs& g, int nacc) {
-    int maxN = 0;
-    for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
-    if (!g.buf_ok || js.empty() || gemm_pipe_kind<R>(js, 1) >= 0 ||
-        gemm_tile(g.nx, maxN, js.size(), sizeof(R) == 4 || nacc == 1) >= GT_H)
-        return {js};
-    std::vector<std::vector<FbJobT<R>>> gr(3), out;
+    if (js.empty() || gemm_pipe_kind<R>(js, g.buf_ok) >= 0) return {js};
+    std::vector<std::vector<FbJobT<R>>> gr(2);
     for (const auto& j : js) {
-        const int k = gemm_pipe_kind<R>({j}, 1);
-        gr[k < 0 ? 2 : k & 1].push_back(j);
+        const int k = gemm_pipe_kind<R>({j}, g.buf_ok);
+        if (k < 0) return {js};
+        gr[k & 1].push_back(j);
     }
-    for (auto& v : gr)
-        if (!v.empty()) out.push_back(std::move(v));
-    return out;
+    if (gemm_piped<R>(gr[0], g, nacc) || gemm_piped<R>(gr[1], g, nacc)) return gr;
+    return {js};
 }
 
 template <>
@@ -1126,8 +1153,7 @@ int32_t launch_fb_gemm<double>(const std::vector<FbJob>& jobs, const FbGemmArgs&
             if (js.empty()) continue;
             // the jobs of two segments first, so that the last blocks to start are short
             std::stable_sort(js.begin(), js.end(), [](const FbJob& a, const FbJob& b) { return a.nseg > b.nseg; });
-            int maxN = 0;
-            for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
+            const int maxN = max_cols(js);
             const FbJob* dj = static_cast<const FbJob*>(device_table(js.data(), js.size() * sizeof(FbJob)));
             if (!dj) return ST_ENOMEM;
             g.pipe = gemm_pipe_kind<double>(js, g.buf_ok);
@@ -1925,14 +1951,6 @@ static int32_t launch_gemm_variant_bf16(const FbJobT<float>* dj, size_t njobs, i
     return ST_OK;
 }
 
-// The split of the matrices is a launch more: for launches of at least 2^29
-// products of a real by a complex value (forward transform, matrices split in
-// the kernel and once per call, microseconds of the whole call, FFT included:
-// 1024 x 128 x 2 modes 29 and 31, 2048 x 128 x 2 39 and 40, 1024 x 256 x 3, 6e8
-// products, 66 and 54, 1024 x 500 x 2 114 and 77; Poisson correction 2048 x 128 x 2
-// 49 and 55, 4096 x 128 x 3 101 and 70).
-constexpr int64_t GEMM_SPLIT_WORK = (int64_t)1 << 29;
-
 template <>
 int32_t launch_fb_gemm<float>(const std::vector<FbJobT<float>>& jobs, const FbGemmArgs& g_in, int family) {
     if (jobs.empty()) return ST_OK;
@@ -1951,16 +1969,10 @@ int32_t launch_fb_gemm<float>(const std::vector<FbJobT<float>>& jobs, const FbGe
             // the jobs of two segments first, so that the last blocks to start are short
             std::stable_sort(js.begin(), js.end(),
                              [](const FbJobT<float>& a, const FbJobT<float>& b) { return a.nseg > b.nseg; });
-            int maxN = 0;
-            for (const auto& j : js) maxN = j.Ncol > maxN ? j.Ncol : maxN;
-            g.pipe = g_mixed_gemm.load() == MIXED_GEMM_BF16X6 ? gemm_pipe_kind<float>(js, g.buf_ok) : -1;
-            if (g.pipe >= 0) {
-                int64_t work = 0;
-                for (const auto& j : js) work += (int64_t)j.nseg * j.K * j.Ncol * g.nx;
-                g.split = nullptr;
-                if (work >= GEMM_SPLIT_WORK) CH_TRY(split_matrices(js, g.split));
-                if (!g.split) g.pipe = -1;
-            }
+            const int maxN = max_cols(js);
+            g.pipe = -1, g.split = nullptr;
+            if (gemm_piped<float>(js, g, pass + 1)) CH_TRY(split_matrices(js, g.split));
+            if (g.split) g.pipe = gemm_pipe_kind<float>(js, g.buf_ok);
             const FbJobT<float>* dj =
                 static_cast<const FbJobT<float>*>(device_table(js.data(), js.size() * sizeof(FbJobT<float>)));
             if (!dj) return ST_ENOMEM;
