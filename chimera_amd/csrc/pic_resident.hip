@@ -169,11 +169,12 @@ __global__ void __launch_bounds__(GP_T) k_gather_push(const double* __restrict__
 //     planes: Re of mode 0, then Re and Im of each mode) with ds_add_f64, the
 //     waves one after the other.  rho follows J through the same LDS.
 //  3. The block hands the tile on:
-//      * a tile of at most DEP_SLOT values goes with plain stores, as it is,
-//        into the group's own slot, with a descriptor (first node row, first
-//        node column, width, rows); k_dep_combine then adds the slots into the
-//        grid, so no global atomics;
-//      * a larger tile is added to the grid with one global atomic per node
+//      * a tile of at most DEP_SLOT values and no more rows than columns (or
+//        DEP_SLOT_R) goes with plain stores, as it is, into the group's own
+//        slot, with a descriptor (first node row, first node column, width,
+//        rows); k_dep_combine then adds the slots into the grid, so no global
+//        atomics;
+//      * any other tile is added to the grid with one global atomic per node
 //        value; the planes take as many passes as the LDS needs (all four
 //        components at once, J then rho, or one component at a time);
 //      * a box with no room even for one component's planes (a group that
@@ -222,6 +223,13 @@ constexpr int DEP_POOL = 2400;
 // values of a slot: at two modes 341 nodes, more than the 65 x 4 of a sparse
 // bunch's 256 particles (4 per cell, drifting over a row boundary)
 constexpr int DEP_SLOT = 4096;
+// node rows of a slot that is narrower than that (others: no more rows than
+// columns, so 64 at most).  A tall, narrow tile (particles column by column, as a
+// RandCell species draws them) is cheaper as global atomics: a wave of the combine would
+// meet a slot of two columns for each of its 64 (65536 particles, 16 per cell in
+// 128 x 32 cells, FP64, the whole deposit: two modes 118 us with slots and 65
+// without, four modes 153 and 70, eight modes 800 and 97).
+constexpr int DEP_SLOT_R = 4;
 constexpr uint32_t DEP_SKIP = 0xFFFFFFFFu;
 
 __device__ __forceinline__ void lds_add(double* p, double v) {
@@ -595,7 +603,7 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
         const int64_t pns64 = (PL * nn64 + 1) & ~(int64_t)1;        // values per component, even
         // components per pass; 0: no tile
         const int per = nc * pns64 <= DEP_POOL ? nc : 3 * pns64 <= DEP_POOL ? 3 : pns64 <= DEP_POOL ? 1 : 0;
-        const bool tiled = per > 0, slotted = tiled && nc * pns64 <= DEP_SLOT;
+        const bool tiled = per > 0, slotted = tiled && TR <= max(DEP_SLOT_R, TX) && nc * pns64 <= DEP_SLOT;
         const int nn = tiled ? (int)nn64 : 1, pns = tiled ? (int)pns64 : 0;
         R* const slot = slotted ? a.slot + (int64_t)grp * DEP_SLOT : nullptr;
         const int rho0 = doJ ? 3 * pns : 0;         // rho in the slot
@@ -657,10 +665,8 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
         }
         if (slotted) {
             d = make_int4(br0, bx0, TX, TR);
-            // (a narrow tile of one or two modes has more rows than the block threads)
-            if (a.mask)
-                for (int r = tid; r < TR; r += DEP_T)
-                    atomicOr(a.mask + (int64_t)(br0 + r) * a.words + (grp >> 11), 1u << ((grp >> 6) & 31));
+            if (a.mask && tid < TR)                 // (TR <= 64)
+                atomicOr(a.mask + (int64_t)(br0 + tid) * a.words + (grp >> 11), 1u << ((grp >> 6) & 31));
         }
     }
     if (tid == 0) a.desc[grp] = d;
