@@ -227,8 +227,8 @@ constexpr int DEP_SLOT = 4096;
 // columns, so 64 at most).  A tall, narrow tile (particles column by column, as a
 // RandCell species draws them) is cheaper as global atomics: a wave of the combine would
 // meet a slot of two columns for each of its 64 (65536 particles, 16 per cell in
-// 128 x 32 cells, FP64, the whole deposit: two modes 118 us with slots and 65
-// without, four modes 153 and 70, eight modes 800 and 97).
+// 128 x 32 cells, FP64, the whole deposit: two modes 118 us with slots and 41
+// without, four modes 153 and 46, eight modes 797 and 55).
 constexpr int DEP_SLOT_R = 4;
 constexpr uint32_t DEP_SKIP = 0xFFFFFFFFu;
 
@@ -683,9 +683,22 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
 // particles.)
 constexpr int CMB_T = 256;
 
+// Instantiations whose sums the compiler would fit into the registers of eight
+// (float) or four (double) waves a SIMD by loading a slot's values one or two at
+// a time, a memory latency each.  They are held to cmb_waves and load all of a
+// slot's values before adding any: 65536 sorted particles, 16 per cell, in 128 x
+// 32 cells, mixed precision: four modes 67 -> 14 us, eight 169 -> 28 (the whole
+// deposit 104 -> 52 and 210 -> 68; before it was one pass 81 and 104).
 template <int NMOD, typename RT>
-__global__ void __launch_bounds__(CMB_T) k_dep_combine(DepArgsT<RT> a, int64_t sr, int64_t sm, int nx1) {
+constexpr bool cmb_batch() { return NMOD >= (sizeof(RT) == 4 ? 4 : 5); }
+template <int NMOD, typename RT>
+constexpr int cmb_waves() { return !cmb_batch<NMOD, RT>() ? 8 : sizeof(RT) == 4 ? 4 : 2; }
+
+template <int NMOD, typename RT>
+__global__ void __launch_bounds__(CMB_T) __attribute__((amdgpu_waves_per_eu(1, cmb_waves<NMOD, RT>())))
+k_dep_combine(DepArgsT<RT> a, int64_t sr, int64_t sm, int nx1) {
     constexpr int PL = 2 * NMOD - 1;
+    constexpr bool BATCH = cmb_batch<NMOD, RT>();
     const int r = blockIdx.y, lane = threadIdx.x & 63;
     const int xs = (blockIdx.x * (CMB_T / 64) + (threadIdx.x >> 6)) * 64, x = xs + lane;
     if (xs >= nx1) return;
@@ -710,16 +723,33 @@ __global__ void __launch_bounds__(CMB_T) k_dep_combine(DepArgsT<RT> a, int64_t s
             if (o >= 0 && o < width) {
                 hit = true;
                 const RT* sp = a.slot + (int64_t)(batch * 64 + j) * DEP_SLOT + (r - row) * width + o;
-                if (doJ) {
+                if constexpr (BATCH) {
+                    RT v[4][PL];
 #pragma unroll
-                    for (int c = 0; c < 3; c++)
+                    for (int c = 0; c < 4; c++) {
+                        if (c < 3 ? !doJ : !doR) continue;
+                        const RT* q = sp + (c < 3 || doJ ? c * pns : 0);
 #pragma unroll
-                        for (int i = 0; i < PL; i++) acc[c][i] += sp[c * pns + i * nn];
-                    sp += 3 * pns;
-                }
-                if (doR) {
+                        for (int i = 0; i < PL; i++) v[c][i] = q[i * nn];
+                    }
 #pragma unroll
-                    for (int i = 0; i < PL; i++) acc[3][i] += sp[i * nn];
+                    for (int c = 0; c < 4; c++) {
+                        if (c < 3 ? !doJ : !doR) continue;
+#pragma unroll
+                        for (int i = 0; i < PL; i++) acc[c][i] += v[c][i];
+                    }
+                } else {
+                    if (doJ) {
+#pragma unroll
+                        for (int c = 0; c < 3; c++)
+#pragma unroll
+                            for (int i = 0; i < PL; i++) acc[c][i] += sp[c * pns + i * nn];
+                        sp += 3 * pns;
+                    }
+                    if (doR) {
+#pragma unroll
+                        for (int i = 0; i < PL; i++) acc[3][i] += sp[i * nn];
+                    }
                 }
             }
         }
