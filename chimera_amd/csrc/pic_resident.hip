@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(GP_T) k_gather_push(const double* __restrict__
 //     planes: Re of mode 0, then Re and Im of each mode) with ds_add_f64, the
 //     waves one after the other.  rho follows J through the same LDS.
 //  3. The block hands the tile on:
-//      * a tile of at most DEP_SLOT values and no more rows than columns (or
+//      * a tile of at most dep_slot values and no more rows than columns (or
 //        DEP_SLOT_R) goes with plain stores, as it is, into the group's own
 //        slot, with a descriptor (first node row, first node column, width,
 //        rows); k_dep_combine then adds the slots into the grid, so no global
@@ -205,7 +205,7 @@ struct DepArgsT {
     GridGeom gJ, gR;    // geometry for J (leftX at the current deposit) and rho
     C* J;               // (nx+1, nr+1, M, 3) or null
     C* R;               // (nx+1, nr+1, M) or null
-    RT* slot;           // [group][DEP_SLOT]: J's components, then rho, each 2M-1 planes of width * rows
+    RT* slot;           // [group][dep_slot]: J's components, then rho, each 2M-1 planes of width * rows
                         // values, starting on an even value
     int4* desc;         // [group]: (first node row or -1, first node column, width, rows)
     uint32_t* mask;     // [nr+1][words]: bit b of a node row: a slot of groups 64b..64b+63 covers it (nullable)
@@ -221,8 +221,10 @@ constexpr int DEP_T = 256, DEP_WAVES = DEP_T / 64;
 // 33 x 2), J on 114 (in the lattice's own order they span 33 x 3).
 constexpr int DEP_POOL = 2400;
 // values of a slot: at two modes 341 nodes, more than the 65 x 4 of a sparse
-// bunch's 256 particles (4 per cell, drifting over a row boundary)
-constexpr int DEP_SLOT = 4096;
+// bunch's 256 particles (4 per cell, drifting over a row boundary); at one mode
+// 528, more than the 257 x 2 of one particle per cell, in half the memory
+// (serve.slot_bytes counts it)
+constexpr int dep_slot(int nmod) { return nmod == 1 ? 2112 : 4096; }
 // node rows of a slot that is narrower than that (others: no more rows than
 // columns, so 64 at most).  A tall, narrow tile (particles column by column, as a
 // RandCell species draws them) is cheaper as global atomics: a wave of the combine would
@@ -603,9 +605,9 @@ __global__ void __launch_bounds__(DEP_T, 3) k_push_deposit(DepArgsT<R> a) {
         const int64_t pns64 = (PL * nn64 + 1) & ~(int64_t)1;        // values per component, even
         // components per pass; 0: no tile
         const int per = nc * pns64 <= DEP_POOL ? nc : 3 * pns64 <= DEP_POOL ? 3 : pns64 <= DEP_POOL ? 1 : 0;
-        const bool tiled = per > 0, slotted = tiled && TR <= max(DEP_SLOT_R, TX) && nc * pns64 <= DEP_SLOT;
+        const bool tiled = per > 0, slotted = tiled && TR <= max(DEP_SLOT_R, TX) && nc * pns64 <= dep_slot(NMOD);
         const int nn = tiled ? (int)nn64 : 1, pns = tiled ? (int)pns64 : 0;
-        R* const slot = slotted ? a.slot + (int64_t)grp * DEP_SLOT : nullptr;
+        R* const slot = slotted ? a.slot + (int64_t)grp * dep_slot(NMOD) : nullptr;
         const int rho0 = doJ ? 3 * pns : 0;         // rho in the slot
         const int64_t corner = bx0 + br0 * sr;      // grid node of the tile's first node
         auto keys = [&](const bool (&ok)[PPL], const int (&ix)[PPL], const int (&ir)[PPL], uint32_t (&key)[PPL])
@@ -722,7 +724,7 @@ k_dep_combine(DepArgsT<RT> a, int64_t sr, int64_t sm, int nx1) {
             const int nn = width * rows, pns = (PL * nn + 1) & ~1, o = x - col;
             if (o >= 0 && o < width) {
                 hit = true;
-                const RT* sp = a.slot + (int64_t)(batch * 64 + j) * DEP_SLOT + (r - row) * width + o;
+                const RT* sp = a.slot + (int64_t)(batch * 64 + j) * dep_slot(NMOD) + (r - row) * width + o;
                 if constexpr (BATCH) {
                     RT v[4][PL];
 #pragma unroll
@@ -1092,7 +1094,7 @@ static int32_t push_deposit_impl(double* coord, double* coord_half, const R* mom
     const int nbatch = (a.ngroups + 63) / 64;
     a.words = (nbatch + 31) / 32;
     const size_t mask_bytes = nbatch > 16 ? (size_t)(nr + 1) * a.words * sizeof(uint32_t) : 0;
-    a.slot = static_cast<R*>(scratch(16, (size_t)a.ngroups * DEP_SLOT * sizeof(R)));
+    a.slot = static_cast<R*>(scratch(16, (size_t)a.ngroups * dep_slot(nkO + 1) * sizeof(R)));
     a.desc = static_cast<int4*>(scratch(18, (size_t)a.ngroups * sizeof(int4)));
     a.mask = mask_bytes ? static_cast<uint32_t*>(scratch(19, mask_bytes)) : nullptr;
     if (!a.slot || !a.desc || (mask_bytes && !a.mask)) return ST_ENOMEM;

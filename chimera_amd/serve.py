@@ -41,9 +41,17 @@ from .diagnostics import Diagnostics
 GIB = 1 << 30
 
 
+def slot_bytes(n, cells, modes, precision="fp64"):
+    """Scratch memory of the deposit of n particles on a grid of `cells` cells: a
+    slot of a group's node sums (dep_slot values, pic_resident.hip) for each group
+    of 512 particles where they average 8 or more per cell, else of 256."""
+    group = 512 if n >= 8 * cells and n >= 512 * 512 else 256
+    return -(-int(n) // group) * (2112 if modes == 1 else 4096) * (8 if precision == "fp64" else 4)
+
+
 def estimate_bytes(spec, precision="fp64"):
     """Device memory a workload needs, from its grid and particle counts, with a
-    1.5x margin for capacity growth and scratch memory."""
+    1.5x margin for capacity growth and scratch memory, and the deposit's slots."""
     s = spec["solver"]
     xmin, xmax, rmax, dx, dr = s["Grid"]
     Nx = int(round((xmax - xmin) / dx))
@@ -61,7 +69,7 @@ def estimate_bytes(spec, precision="fp64"):
         fc = spec["electrons"]["FixedCell"]
         n = Nx * Nkr * int(np.prod(fc))
         parts = 2 * n * (48 + 4 * su)
-    return int(1.5 * (grid + fb + tables + parts))
+    return int(1.5 * (grid + fb + tables + parts)) + slot_bytes(n, Nx * Nkr, M, precision)
 
 
 class Request:

@@ -118,6 +118,21 @@ def test_memory_estimate_scales_with_size():
     assert S.estimate_bytes(big, "mixed") < e1
 
 
+def test_memory_estimate_holds_the_deposit_slots():
+    # one group of 256 particles after the other: a slot of 4096 values each (two modes and more)
+    assert S.slot_bytes(2.6e6, 2048 * 256, 2) == 10157 * 4096 * 8
+    assert S.slot_bytes(2.6e6, 2048 * 256, 1) == 10157 * 2112 * 8
+    assert S.slot_bytes(2.6e6, 512 * 64, 2, "mixed") == 5079 * 4096 * 4      # groups of 512
+    # a sparse bunch (2048 x 256 cells): of each of its 1.3 n_target particles the estimate
+    # holds the particle with its margin and its share of a slot (128 B in FP64)
+    def bunch(n):
+        b = W.beam(2048, 256, 200.0, 10.0, 5.0, 1e-6, 2e6, 2.0, 300.0)
+        return dict(b, params=dict(b["params"], n_target=n))
+    for precision, part, slot in (("fp64", 80, 128), ("mixed", 64, 64)):
+        grown = S.estimate_bytes(bunch(2e6), precision) - S.estimate_bytes(bunch(1e6), precision)
+        assert grown >= 1.3e6 * (1.5 * part + slot) - 4096 * 8 - 1
+
+
 def test_table_cache_returns_read_only_shared_tables():
     kx = 2 * np.pi * np.fft.fftfreq(64, 0.1)
     R = 0.3 * (np.arange(17) - 0.5)
