@@ -987,7 +987,7 @@ static int32_t gemm_tile_launch(const FbJobT<float>* dj, size_t nj, int maxN, co
 //
 // With autotuning on (chimera_set_autotune), the first launch of a GEMM shape
 // -- (element type, GEMM form, accumulators, nx, columns, jobs, K, segments,
-// buffer-load path) -- times every tile shape the form has a kernel for and
+// kernels) -- times every tile shape the form has a kernel for and
 // keeps the fastest for that shape; later launches of the shape use it.  The
 // timed launches run the real job table with every output redirected to a
 // scratch buffer (the operands are only read), three launches per shape after
@@ -998,6 +998,12 @@ static int32_t gemm_tile_launch(const FbJobT<float>* dj, size_t nj, int maxN, co
 // cannot grow, a shape not yet tuned takes the block-count rule (gemm_tile).
 // Every tile shape sums each output over K in the same order, so the choice
 // changes the time of a launch, not its result.
+// The last number of a shape names the kernels that its tiles were timed on: the
+// pipeline for its kind of segments or the general kernels, with or without
+// buffer loads, from TUNE_KERNELS up.  A file of other kernels (it has 0 or 1
+// there) is not used: raise TUNE_KERNELS when they change.
+constexpr int TUNE_KERNELS = 10;
+static int tune_kernels(const FbGemmArgs& g) { return TUNE_KERNELS + 2 * (g.pipe + 1) + g.buf_ok; }
 struct TuneKey {
     int v[9];
     bool operator<(const TuneKey& o) const { return std::lexicographical_compare(v, v + 9, o.v, o.v + 9); }
@@ -1019,7 +1025,7 @@ static void tune_load_locked() {
     double ms;
     while (fscanf(f, "%d %d %d %d %d %d %d %d %d %d %lf", &k.v[0], &k.v[1], &k.v[2], &k.v[3], &k.v[4], &k.v[5],
                   &k.v[6], &k.v[7], &k.v[8], &tile, &ms) == 11)
-        if (tile >= GT_W4 && tile <= GT_Q) g_tuned[k] = tile;
+        if (tile >= GT_W4 && tile <= GT_Q && k.v[8] >= TUNE_KERNELS && k.v[8] < TUNE_KERNELS + 10) g_tuned[k] = tile;
     fclose(f);
 }
 
@@ -1035,7 +1041,7 @@ static int gemm_choose_tile(const J* dj, const std::vector<J>& js, int maxN, con
         nseg = j.nseg > nseg ? j.nseg : nseg;
     }
     const int form = rbytes == 4 ? g_mixed_gemm.load() : 2;
-    const TuneKey key = {{rbytes, form, nacc, g.nx, maxN, (int)nj, maxK, nseg, g.buf_ok}};
+    const TuneKey key = {{rbytes, form, nacc, g.nx, maxN, (int)nj, maxK, nseg, tune_kernels(g)}};
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         tune_load_locked();

@@ -58,9 +58,10 @@ int32_t chimera_set_mixed_gemm(int32_t form);
 int32_t chimera_get_mixed_gemm(void);
 /* Tile autotuner of the Hankel and FB-operator GEMMs (no counterpart in the
  * reference).  on = 1: the first launch of each GEMM shape (element type,
- * form, accumulators, Nx, columns, jobs, K, segments) times every tile shape
+ * form, accumulators, Nx, columns, jobs, K, segments, kernels) times every tile shape
  * and keeps the fastest; on = 0 (default): tiles by a block-count rule.  path
- * (may be NULL) names a text file of tuned shapes, read once and appended to.
+ * (may be NULL) names a text file of tuned shapes, read once and appended to
+ * (shapes timed on other kernels than this library's are passed over).
  * chimera_autotune_entries returns the number of shapes tuned or loaded. */
 int32_t chimera_set_autotune(int32_t on, const char* path);
 int32_t chimera_autotune_entries(void);

@@ -78,3 +78,32 @@ def test_autotuned_tiles_same_bits(gpu, tmp_path):
     finally:
         L.chimera_set_autotune(0, None)
         L.chimera_set_mixed_gemm(old_form)
+
+
+def test_shapes_name_their_kernels(gpu, tmp_path):
+    """The curl's lists of the two kinds of segments go to different kernels: each
+    is timed by itself, and a file of shapes timed on other kernels is not used."""
+    from chimera_amd._lib import lib
+    L = lib()
+    r = rng(4343)
+    nkx, nkr, nko = 8192, 128, 1
+    kx = 2 * np.pi * np.fft.fftfreq(nkx, 0.1)
+    Dp, Dm = F(r, nkr, nkr, nko + 2), F(r, nkr, nkr, nko + 2)
+    v = C(r, nkx, nkr, nko + 1, 3)
+    z3 = np.zeros((nkx, nkr, nko + 1, 3), complex, order="F")
+    path, other = tmp_path / "tiles.txt", tmp_path / "other.txt"
+    try:
+        L.chimera_set_autotune(0, None)
+        ref = gpu.fb_rot(z3.copy(order="F"), v, Dp, Dm, kx)
+        say("case: fb_rot 8192x128 m=0..1, autotuned, fp64")
+        assert L.chimera_set_autotune(1, str(path).encode()) == 0
+        assert np.array_equal(_bits(gpu.fb_rot(z3.copy(order="F"), v, Dp, Dm, kx)), _bits(ref))
+        rows = [ln.split() for ln in path.read_text().splitlines()]
+        assert len({f[8] for f in rows}) > 1, rows
+        n = L.chimera_autotune_entries()
+        other.write_text("".join(" ".join(f[:3] + [str(int(f[3]) + 2)] + f[4:8] + ["1"] + f[9:]) + "\n" for f in rows))
+        assert L.chimera_set_autotune(1, str(other).encode()) == 0
+        gpu.fb_rot(z3.copy(order="F"), v, Dp, Dm, kx)
+        assert L.chimera_autotune_entries() == n
+    finally:
+        L.chimera_set_autotune(0, None)
