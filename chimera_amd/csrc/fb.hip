@@ -119,30 +119,27 @@ __device__ __forceinline__ float2 seg_finish(const FbSegT<float>& s, float2 v0, 
 // every stage.)
 constexpr int GB_LDK = GB_K + 1;
 
-// One K-stage (GB_K = 16) of a wave's (16*NI) x (16*WN) tile: NI x WN MFMA
-// tiles (NI = 4 for 64-complex x tiles, 2 for 32-complex ones).
-template <int WN, int NI>
-__device__ __forceinline__ void mfma_stage(dbl4 (&acc)[NI][WN], const double* __restrict__ As,
+// One K-stage (GB_K = 16) of a wave's (16*NI) x 16 tile: NI MFMA tiles (NI = 2
+// for 32-complex x tiles, 1 for 16-complex ones).
+template <int NI>
+__device__ __forceinline__ void mfma_stage(dbl4 (&acc)[NI][1], const double* __restrict__ As,
                                            const double* __restrict__ Ds, int lane, int wr, int wc) {
     constexpr int LDA = 32 * NI + GB_PAD;
 #pragma unroll
     for (int kq = 0; kq < GB_K / 4; kq++) {
         const int kk = kq * 4 + (lane >> 4);
-        double a[NI], b[WN];
+        double a[NI];
 #pragma unroll
         for (int i = 0; i < NI; i++) a[i] = As[kk * LDA + wr * 16 * NI + i * 16 + (lane & 15)];
+        const double b = Ds[(wc * 16 + (lane & 15)) * GB_LDK + kk];
 #pragma unroll
-        for (int j = 0; j < WN; j++) b[j] = Ds[(wc * 16 * WN + j * 16 + (lane & 15)) * GB_LDK + kk];
-#pragma unroll
-        for (int i = 0; i < NI; i++)
-#pragma unroll
-            for (int j = 0; j < WN; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < NI; i++) acc[i][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b, acc[i][0], 0, 0, 0);
     }
 }
 
-// LDS bytes of one k_fb_gemm<NACC, WN, GX> block: A and D stages, double-buffered.
-constexpr size_t gb_lds_bytes(int WN, int GX) {
-    return 2 * ((size_t)GB_K * (2 * GX + GB_PAD) + (size_t)32 * WN * GB_LDK) * sizeof(double);
+// LDS bytes of one k_fb_gemm<NACC, GX> block: A and D stages, double-buffered.
+constexpr size_t gb_lds_bytes(int GX) {
+    return 2 * ((size_t)GB_K * (2 * GX + GB_PAD) + (size_t)32 * GB_LDK) * sizeof(double);
 }
 
 // Fast-path loads of the K-stages.  With the thread layout of the fetch
@@ -192,8 +189,9 @@ __device__ __forceinline__ bool seg_plain(const FbSegT<R>& S) {
 
 // Output elements per batch of the epilogue, by element type and accumulator
 // registers (a batch holds up to seven loaded values and an offset per element).
+// (FP64: tiles of 32 columns alone, wn = 1.)
 constexpr int gemm_eb(int rbytes, int nacc, int wn) {
-    return rbytes == 4 ? (nacc * wn <= 2 ? 8 : nacc * wn == 4 ? 4 : 2) : (nacc * wn <= 2 ? 4 : wn == 4 ? 1 : 2);
+    return rbytes == 8 ? 4 : nacc * wn <= 2 ? 8 : nacc * wn == 4 ? 4 : 2;
 }
 
 // Epilogue of both GEMM kernels.  For row tile i, column tile j and h = 0, 1 a
@@ -210,19 +208,18 @@ __device__ __forceinline__ void gemm_epilogue_serial(const FbJobT<R>& J, const F
                                                      const ACC (&acc1)[NI][NACC == 2 ? WN : 1], int Ncol, int n0,
                                                      int x0, int lane, int wr, int wc);
 
-template <typename R, int NACC, int WN, int NI, int EBM = 8, typename ACC>
+template <typename R, int NACC, int WN, int NI, typename ACC>
 __device__ __forceinline__ void gemm_epilogue(const FbJobT<R>& J, const FbGemmArgs& g, const ACC (&acc0)[NI][WN],
                                               const ACC (&acc1)[NI][NACC == 2 ? WN : 1], int Ncol, int n0, int x0,
                                               int lane, int wr, int wc) {
     if constexpr (WN == 4) {
-        // the 128-column tiles of large grids have no registers to spare for a
+        // (FP32) the 128-column tiles of large grids have no registers to spare for a
         // batch; their launches have enough blocks to hide the latency
         gemm_epilogue_serial<R, NACC, WN, NI>(J, g, acc0, acc1, Ncol, n0, x0, lane, wr, wc);
         return;
     }
     typedef cplx_t<R> C;
-    constexpr int NE = NI * WN * 2, EB0 = gemm_eb((int)sizeof(R), NACC, WN), EB1 = EB0 < EBM ? EB0 : EBM;
-    constexpr int EB = EB1 < NE ? EB1 : NE;
+    constexpr int NE = NI * WN * 2, EB0 = gemm_eb((int)sizeof(R), NACC, WN), EB = EB0 < NE ? EB0 : NE;
     static_assert(NE % EB == 0, "epilogue batch");
     const int nout = J.nout;
     const bool beta = J.beta != 0;
@@ -328,15 +325,15 @@ __device__ __forceinline__ void gemm_epilogue_serial(const FbJobT<R>& J, const F
 }
 
 // The tiles of 32 and 16 complex x (GX), for small grids, and any launch that
-// k_fb_gemm_pipe does not take.  Block tile: GX complex x (2*GX real rows) x
-// 32*WN columns; 4 waves as 2 x 2, each GX rows x 16*WN columns.  NACC = 2 keeps a second accumulator set,
-// fed by segment 1 (launch_fb_gemm orders the segments so).  The K-stages of
+// k_fb_gemm_pipe does not take.  Block tile: GX complex x (2*GX real rows) x 32
+// columns; 4 waves as 2 x 2, each GX rows x 16 columns.  NACC = 2 keeps a second
+// accumulator set, fed by segment 1 (launch_fb_gemm orders the segments so).  The K-stages of
 // all segments form one pipeline: the global loads of stage t+1 go to
 // registers while the MFMAs of stage t run, then land in the other LDS
 // buffer, with one barrier per stage.
-template <int NACC, int WN, int GX>
+template <int NACC, int GX>
 __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm(const FbJob* __restrict__ jobs, FbGemmArgs g) {
-    constexpr int NI = GX / 16, BN = 32 * WN, LDA = 2 * GX + GB_PAD;
+    constexpr int NI = GX / 16, BN = 32, LDA = 2 * GX + GB_PAD;
     constexpr int A_STAGE = GB_K * LDA, D_STAGE = BN * GB_LDK;
     const FbJob& J = jobs[blockIdx.z];
     const int Ncol = J.Ncol, K = J.K, nseg = J.nseg;
@@ -349,11 +346,9 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm(const FbJob* __restri
     double* const As = gb_smem;                  // [2][GB_K][LDA]
     double* const Ds = gb_smem + 2 * A_STAGE;    // [2][BN][GB_LDK]
 
-    dbl4 acc0[NI][WN], acc1[NI][NACC == 2 ? WN : 1];
+    dbl4 acc0[NI][1], acc1[NI][1];
 #pragma unroll
-    for (int i = 0; i < NI; i++)
-#pragma unroll
-        for (int j = 0; j < WN; j++) acc0[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+    for (int i = 0; i < NI; i++) acc0[i][0] = dbl4{0.0, 0.0, 0.0, 0.0};
 
     constexpr int NA = (GB_K * GX) / GB_THREADS, ND = (GB_K * BN) / GB_THREADS;
     const int stages_per_seg = (K + GB_K - 1) / GB_K;
@@ -442,10 +437,10 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm(const FbJob* __restri
     };
     // K-stages [tb, te) into one accumulator set; the prefetch runs across the
     // boundary between the two segments of a two-accumulator job
-    auto pipe = [&](dbl4 (&acc)[NI][WN], int tb, int te) __attribute__((always_inline)) {
+    auto pipe = [&](dbl4 (&acc)[NI][1], int tb, int te) __attribute__((always_inline)) {
         for (int t = tb; t < te; t++) {
             if (t + 1 < nstages) fetch(t + 1);
-            mfma_stage<WN, NI>(acc, As + (t & 1) * A_STAGE, Ds + (t & 1) * D_STAGE, lane, wr, wc);
+            mfma_stage<NI>(acc, As + (t & 1) * A_STAGE, Ds + (t & 1) * D_STAGE, lane, wr, wc);
             if (t + 1 < nstages) stash((t + 1) & 1, t + 1);
             __syncthreads();
         }
@@ -458,14 +453,12 @@ __global__ void __launch_bounds__(GB_THREADS, 2) k_fb_gemm(const FbJob* __restri
     if constexpr (NACC == 2) {
         pipe(acc0, 0, nseg > 0 ? stages_per_seg : 0);   // a job without segments stages nothing
 #pragma unroll
-        for (int i = 0; i < NI; i++)
-#pragma unroll
-            for (int j = 0; j < WN; j++) acc1[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+        for (int i = 0; i < NI; i++) acc1[i][0] = dbl4{0.0, 0.0, 0.0, 0.0};
         pipe(acc1, stages_per_seg, nstages);
     } else {
         pipe(acc0, 0, nstages);
     }
-    gemm_epilogue<double, NACC, WN, NI>(J, g, acc0, acc1, Ncol, n0, x0, lane, wr, wc);
+    gemm_epilogue<double, NACC, 1, NI>(J, g, acc0, acc1, Ncol, n0, x0, lane, wr, wc);
 }
 
 // ---- tiles of 64 complex x: a software pipeline
@@ -814,17 +807,17 @@ static int32_t launch_gemm_pipe(const FbJob* dj, size_t njobs, int maxN, const F
     }
 }
 
-template <int NACC, int WN, int GX>
+template <int NACC, int GX>
 static int32_t launch_gemm_variant(const FbJob* dj, size_t njobs, int maxN, const FbGemmArgs& g) {
-    constexpr int BN = 32 * WN;
+    constexpr int BN = 32;
     static bool attr = false;
     if (!attr) {
-        CH_HIP(hipFuncSetAttribute((const void*)k_fb_gemm<NACC, WN, GX>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)gb_lds_bytes(WN, GX)));
+        CH_HIP(hipFuncSetAttribute((const void*)k_fb_gemm<NACC, GX>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)gb_lds_bytes(GX)));
         attr = true;
     }
     dim3 grid((unsigned)((g.nx + GX - 1) / GX), (unsigned)((maxN + BN - 1) / BN), (unsigned)njobs);
-    hipLaunchKernelGGL((k_fb_gemm<NACC, WN, GX>), grid, GB_THREADS, gb_lds_bytes(WN, GX), stream(), dj, g);
+    hipLaunchKernelGGL((k_fb_gemm<NACC, GX>), grid, GB_THREADS, gb_lds_bytes(GX), stream(), dj, g);
     CH_LAUNCH_CHECK("k_fb_gemm");
     return ST_OK;
 }
@@ -924,16 +917,16 @@ static int32_t gemm_tile_launch(const FbJob* dj, size_t nj, int maxN, const FbGe
             case GT_W4: return launch_gemm_pipe<1, 4>(dj, nj, maxN, g);
             case GT_W2: return launch_gemm_pipe<1, 2>(dj, nj, maxN, g);
             case GT_W1: return launch_gemm_pipe<1, 1>(dj, nj, maxN, g);
-            case GT_H: return launch_gemm_variant<1, 1, GB_X / 2>(dj, nj, maxN, g);
-            default: return launch_gemm_variant<1, 1, GB_X / 4>(dj, nj, maxN, g);
+            case GT_H: return launch_gemm_variant<1, GB_X / 2>(dj, nj, maxN, g);
+            default: return launch_gemm_variant<1, GB_X / 4>(dj, nj, maxN, g);
         }
     }
     switch (tile) {
         case GT_W4: return ST_EUNSUP;
         case GT_W2: return launch_gemm_pipe<2, 2>(dj, nj, maxN, g);
         case GT_W1: return launch_gemm_pipe<2, 1>(dj, nj, maxN, g);
-        case GT_H: return launch_gemm_variant<2, 1, GB_X / 2>(dj, nj, maxN, g);
-        default: return launch_gemm_variant<2, 1, GB_X / 4>(dj, nj, maxN, g);
+        case GT_H: return launch_gemm_variant<2, GB_X / 2>(dj, nj, maxN, g);
+        default: return launch_gemm_variant<2, GB_X / 4>(dj, nj, maxN, g);
     }
 }
 
