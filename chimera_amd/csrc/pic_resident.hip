@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(GP_T) k_gather_push(const double* __restrict__
 // What bounds it: about equally the 104 bytes per particle in and out of HBM
 // (with the slots 8.9 GB of traffic for 67.0 M electrons at four modes), the
 // segments' arithmetic and their LDS reads and adds; three blocks of a CU share
-// them.  There it takes 3.1 ms (2.8 without the fixed order of the adds), and the
+// them.  There it takes 3.0 ms (2.8 without the fixed order of the adds), and the
 // combine 0.9; one pass per component over particles re-read from memory (46 GB)
 // took 5.5, with a combine of 1.2.  Mixed precision, 16.7 M at three modes: 0.82 +
 // 0.11 ms, before 1.24 + 0.13 and 70 us to sort the slots.  (Loading the next group during the deposit of one, a

@@ -132,12 +132,14 @@ def test_deposit_paths(port, nx, nkr, nko, n, order, precision):
     check(port, coord, half, coord, mom, w, g, out, precision, shift=0.03)
 
 
-# Tiles of two or three node columns and more node rows than a group has
-# threads, with row masks (more than 1024 groups of 256 particles): every row of
-# such a tile must be marked.  "randcell": the order of Species.gen_randcell with
+# Tiles of two or three node columns and hundreds of node rows, most of them more
+# than a group has threads, with row masks (more than 1024 groups of 256
+# particles) and without: no row of such a tile may be lost, whichever way it goes
+# to the grid (all components at once, J then rho, one at a time).  "randcell": the order of Species.gen_randcell with
 # one particle a cell (column by column, the radius fastest); "sheet": one column
 # of cells, its particles in random order.
 @pytest.mark.parametrize("nx,nkr,nko,n,order,curr", [(1025, 299, 0, 1024 * 299, "randcell", True),
+                                                     (1025, 250, 0, 1024 * 250, "randcell", True),
                                                      (201, 500, 0, 600000, "sheet", True),
                                                      (201, 390, 1, 600000, "sheet", False)])
 def test_deposit_tall_tiles(port, nx, nkr, nko, n, order, curr):
@@ -176,8 +178,8 @@ def test_deposit_push_and_parts(port, curr, dens, ld_extra):
 
 def test_deposit_skips_and_lost_particles(port):
     """Particles outside the grid (the reference would write outside its
-    arrays), not a number, at rest or without weight deposit nothing; nothing
-    else changes."""
+    arrays) or not a number deposit nothing; nothing else changes.  (At rest and
+    without weight: test_deposit_paths, whose particles have both.)"""
     say("case: skipped particles")
     g = Grid(nx=33, nkr=9, nko=2, leftX=-1.65)
     coord, mom, w = particles(g, 900, seed=8)
